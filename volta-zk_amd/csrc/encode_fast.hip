@@ -118,7 +118,7 @@ template <bool LATE>
 __device__ __forceinline__ void encode_rows(int S, const int16_t* __restrict__ w, size_t cols, size_t rows,
                                             const uint64_t* __restrict__ grid, const v4i* __restrict__ frags,
                                             const v4i* __restrict__ init, uint64_t* __restrict__ out, uint64_t* Y,
-                                            int lane, uint32_t k16, uint32_t keps) {
+                                            int lane, uint32_t k16) {
     constexpr int NP = enc13m::PAIRS;
     int H = 1 - (S & 1);
     const int j1b = (S >> 1) * 64 + lane;
@@ -200,7 +200,7 @@ __device__ __forceinline__ void encode_rows(int S, const int16_t* __restrict__ w
             for (int t = 0; t < 4; ++t) {
                 const int a[4] = {d[P][t][0][0], d[P][t][0][1], d[P][t][0][2], d[P][t][0][3]};
                 const int b[4] = {d[P][t][1][0], d[P][t][1][1], d[P][t][1][2], d[P][t][1][3]};
-                y[t] = gl::mul32x4(enc13m::recombine(a, b, k16, keps), g[P][t]);
+                y[t] = gl::mul32x4(enc13m::recombine(a, b, k16), g[P][t]);
             }
             // columns i2 = 16 t + m and i2 + 32 (t + 2) of row j1 are both in
             // this lane: store phase B's first-stage sums and differences
@@ -223,13 +223,13 @@ __device__ __forceinline__ void encode_rows(int S, const int16_t* __restrict__ w
 template <bool LATE>
 __global__ __launch_bounds__(THREADS, 2) void encode13_i16(const int16_t* __restrict__ w, size_t cols, size_t rows,
                                                           const uint64_t* __restrict__ tables,
-                                                          uint64_t* __restrict__ out, uint32_t k16, uint32_t keps) {
+                                                          uint64_t* __restrict__ out, uint32_t k16) {
     extern __shared__ uint64_t Y[];
     const int lane = threadIdx.x & 63;
     const v4i* frags = reinterpret_cast<const v4i*>(reinterpret_cast<const unsigned char*>(tables) + GRID_BYTES);
     const v4i* init = reinterpret_cast<const v4i*>(reinterpret_cast<const unsigned char*>(frags) + enc13m::FRAG_BYTES);
-    encode_rows<LATE>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w, cols, rows, tables, frags, init, out, Y, lane, k16,
-                keps);
+    encode_rows<LATE>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w, cols, rows, tables, frags, init, out, Y, lane,
+                      k16);
 }
 
 // grid[j1 * 64 + i2] = w^(i2 j1) from the half table (w^e = -w^(e - n/2)).
@@ -292,10 +292,10 @@ int encode_i16_fast(Context* c, const int16_t* w, size_t rows, size_t cols, size
     const uint64_t* grid = t->grid;
     if (late)
         hipLaunchKernelGGL(enc13::encode13_i16<true>, dim3(blocks), dim3(enc13::THREADS), enc13::LDS_BYTES, c->stream,
-                           w, cols, rows, grid, out, 65536u, 0xFFFFFFFFu);
+                           w, cols, rows, grid, out, 65536u);
     else
         hipLaunchKernelGGL(enc13::encode13_i16<false>, dim3(blocks), dim3(enc13::THREADS), enc13::LDS_BYTES, c->stream,
-                           w, cols, rows, grid, out, 65536u, 0xFFFFFFFFu);
+                           w, cols, rows, grid, out, 65536u);
     VMX_HIP(c, hipGetLastError());
     return 0;
 }

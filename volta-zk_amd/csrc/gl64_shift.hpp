@@ -21,36 +21,56 @@ namespace gl {
 constexpr int E_W64 = 39;  // w_64 = 2^39
 constexpr int E_W32 = 78;  // w_32 = 2^78
 
-// x * 2^-M mod p for 1 <= M <= 32, x canonical; canonical result.
+// x << S and x >> S as one 64-bit instruction on the device, where the compiler
+// would take two 32-bit ones when it needs the halves apart.
+template <int S>
+__host__ __device__ __forceinline__ uint64_t shl64(uint64_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (S > 0 && S < 32) {
+        uint64_t r;
+        asm("v_lshlrev_b64 %0, %1, %2" : "=v"(r) : "n"(S), "v"(x));
+        return r;
+    }
+#endif
+    return x << S;
+}
+template <int S>
+__host__ __device__ __forceinline__ uint64_t shr64(uint64_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (S > 0 && S < 32) {
+        uint64_t r;
+        asm("v_lshrrev_b64 %0, %1, %2" : "=v"(r) : "n"(S), "v"(x));
+        return r;
+    }
+#endif
+    return x >> S;
+}
+
+// The multiplications by a power of two below take any u64 and give a
+// canonical result.
+
+// x * 2^-M mod p for 1 <= M <= 32.
 // With x = q 2^M + r (r < 2^M): x 2^-M = q + r 2^-M and 2^-M = -2^(96-M), so
 // x 2^-M = q - r 2^(32-M) 2^64 = q - r' eps with r' = r 2^(32-M) < 2^32; both
 // q < 2^(64-M) and r' eps <= (2^32-1)^2 are canonical.
 template <int M>
 __host__ __device__ __forceinline__ uint64_t shr_mod(uint64_t x) {
     static_assert(M >= 1 && M <= 32, "shift out of range");
-    const uint64_t q = x >> M;
+    const uint64_t q = shr64<M>(x);
     const uint32_t rp = static_cast<uint32_t>(x) << (32 - M);
     return sub(q, static_cast<uint64_t>(rp) * EPS);
 }
 
-// x * 2^(32+SM) mod p for 0 <= SM < 32, x canonical; canonical result.
+// x * 2^(32+SM) mod p for 0 <= SM < 32.
 // In 32-bit words x 2^SM = W1 + W2 2^32 + W3 2^64, so x 2^(32+SM) =
 // W1 2^32 + W2 2^64 + W3 2^96 = (W1 + W2) 2^32 - (W2 + W3)  (2^64 = 2^32 - 1,
 // 2^96 = -1): two 32-bit sums and one borrow-corrected 64-bit difference.
 template <int SM>
 __host__ __device__ __forceinline__ uint64_t shl_mod_hi(uint64_t x) {
     static_assert(SM >= 0 && SM < 32, "shift out of range");
-    const uint32_t x0 = static_cast<uint32_t>(x), x1 = static_cast<uint32_t>(x >> 32);
-    uint32_t w1, w2, w3;
-    if constexpr (SM == 0) {
-        w1 = x0;
-        w2 = x1;
-        w3 = 0;
-    } else {
-        w1 = x0 << SM;
-        w2 = (x1 << SM) | (x0 >> (32 - SM));
-        w3 = x1 >> (32 - SM);
-    }
+    const uint64_t xs = shl64<SM>(x);
+    const uint32_t w1 = static_cast<uint32_t>(xs), w2 = static_cast<uint32_t>(xs >> 32);
+    const uint32_t w3 = SM == 0 ? 0u : static_cast<uint32_t>(x >> 32) >> ((32 - SM) & 31);
     unsigned ca, cb, c2, b0, b1;
     const uint32_t a = __builtin_addc(w1, w2, 0u, &ca);  // A = a + ca 2^32
     const uint32_t b = __builtin_addc(w2, w3, 0u, &cb);  // B = b + cb 2^32 < 2^32 + 2^31
@@ -59,11 +79,32 @@ __host__ __device__ __forceinline__ uint64_t shl_mod_hi(uint64_t x) {
     const uint32_t chi = cb | c2;
     const uint32_t r0 = __builtin_subc(0u, clo, 0u, &b0);  // r = h 2^32 - C
     const uint32_t r1 = __builtin_subc(h, chi, b0, &b1);
-    const uint64_t r = pack64(r0, r1);
-    return b1 ? r - EPS : r;  // negative: + p = - eps mod 2^64
+    return less_eps(pack64(r0, r1), b1 != 0);  // negative: + p = - eps mod 2^64
 }
 
-// x * 2^S mod p for 0 <= S < 96, x canonical; canonical result.
+// -(x * 2^(32+SM)) mod p for 0 <= SM < 32.
+// With the words of x 2^SM as in shl_mod_hi, the value is (W2 + W3) - (W1 + W2) X
+// (X = 2^32).  W1 + W2 = s + cs X and cs X^2 = cs (X - 1), so it is
+// L - h X with h = s + cs < 2^32 (no carry: cs = 1 leaves s <= 2^32 - 2) and
+// L = W2 + W3 + cs = l0 + cl X: the word l0 and the difference cl - h, formed as
+// 1 - h - (1 - cl) so that one subtract-with-borrow takes both.  A borrow means
+// a negative value: + p, i.e. - eps mod 2^64.  Two shifts and six VALU
+// instructions, against ten for the positive value.
+template <int SM>
+__host__ __device__ __forceinline__ uint64_t shl_mod_hi_neg(uint64_t x) {
+    static_assert(SM >= 0 && SM < 32, "shift out of range");
+    const uint64_t xs = shl64<SM>(x);
+    const uint32_t w1 = static_cast<uint32_t>(xs), w2 = static_cast<uint32_t>(xs >> 32);
+    const uint32_t w3 = SM == 0 ? 0u : static_cast<uint32_t>(x >> 32) >> ((32 - SM) & 31);
+    unsigned cs, none, cl, b;
+    const uint32_t s = __builtin_addc(w1, w2, 0u, &cs);
+    const uint32_t h = __builtin_addc(s, 0u, cs, &none);
+    const uint32_t l0 = __builtin_addc(w2, w3, cs, &cl);
+    const uint32_t hi = __builtin_subc(1u, h, cl ? 0u : 1u, &b);
+    return less_eps(pack64(l0, hi), b != 0);
+}
+
+// x * 2^S mod p for 0 <= S < 96 (S = 0: x itself, canonical if x is).
 template <int S>
 __host__ __device__ __forceinline__ uint64_t shl_mod(uint64_t x) {
     static_assert(S >= 0 && S < 96, "shift out of range");
@@ -79,72 +120,53 @@ __host__ __device__ __forceinline__ uint64_t shl_mod(uint64_t x) {
     }
 }
 
-// -(x * 2^S) mod p for 64 <= S < 96 without the final negation.
+// -(x * 2^S) mod p for 32 <= S < 96, whose negative is the cheaper form.
 template <int S>
 __host__ __device__ __forceinline__ uint64_t shl_mod_neg(uint64_t x) {
-    static_assert(S >= 64 && S < 96, "only the division form has a cheap negative");
-    return shr_mod<96 - S>(x);
+    static_assert(S >= 32 && S < 96, "no cheap negative below 2^32");
+    if constexpr (S < 64) return shl_mod_hi_neg<S - 32>(x);
+    else return shr_mod<96 - S>(x);
 }
 
-// x * 2^E up to sign, in its cheapest form: with S = (E mod 192) mod 96,
-// 2^E = +-2^S, and for S >= 64 the division form yields -(x 2^S) directly.
-// pow2_neg(E) tells whether the result holds -(x 2^E) rather than x 2^E.
-constexpr bool pow2_neg(int E) {
-    const int e = E % 192;
-    return (e >= 96) != (e % 96 >= 64);
-}
-
-template <int E>
-__host__ __device__ __forceinline__ uint64_t mul_pow2_signed(uint64_t x) {
-    constexpr int S = (E % 192) % 96;
-    if constexpr (S >= 64) return shr_mod<96 - S>(x);
-    else return shl_mod<S>(x);
-}
-
-// x * 2^E mod p for any E >= 0.
+// x * 2^E mod p for any E >= 0: with S = (E mod 192) mod 96, 2^E = +-2^S.
 template <int E>
 __host__ __device__ __forceinline__ uint64_t mul_pow2(uint64_t x) {
-    const uint64_t t = mul_pow2_signed<E>(x);
-    if constexpr (pow2_neg(E)) return neg(t);
-    else return t;
+    constexpr int S = (E % 192) % 96;
+    constexpr bool minus = E % 192 >= 96;
+    if constexpr (S >= 64) {
+        const uint64_t t = shl_mod_neg<S>(x);
+        if constexpr (minus) return t;
+        else return neg(t);
+    } else if constexpr (S >= 32) {
+        if constexpr (minus) return shl_mod_neg<S>(x);
+        else return shl_mod<S>(x);
+    } else {
+        const uint64_t t = shl_mod<S>(x);
+        if constexpr (minus) return neg(t);
+        else return t;
+    }
 }
 
-// DIT butterfly (u, v) <- (u + w v, u - w v) with w = 2^E.
-template <int E>
+// DIT butterfly (u, v) <- (u + w v, u - w v) with w = 2^E, any u64 u, and v any
+// u64 unless the twiddle is trivial (E a multiple of 96), canonical then.  The
+// twiddled value is canonical, so both results take the four-instruction add
+// and sub; an output whose flag (CU, CV: u's, v's new value) is set is
+// canonical, which needs a canonical u.
+template <int E, bool CU = true, bool CV = true>
 __host__ __device__ __forceinline__ void bfly_pow2(uint64_t& u, uint64_t& v) {
-    constexpr int e = E % 192;
-    if constexpr (e == 0) {
-        const uint64_t a = add(u, v), b = sub(u, v);
-        u = a;
-        v = b;
-    } else if constexpr (e == 96) {
-        const uint64_t a = sub(u, v), b = add(u, v);
-        u = a;
-        v = b;
-    } else {
-        // w = +-2^S with S = e mod 96; for S >= 64 the division form yields
-        // -(v 2^S) directly, which flips the sign once more.
-        constexpr int S = e % 96;
-        constexpr bool neg_w = e >= 96;
-        uint64_t t;
-        bool neg_t;
-        if constexpr (S >= 64) {
-            t = shl_mod_neg<S>(v);
-            neg_t = !neg_w;
-        } else {
-            t = shl_mod<S>(v);
-            neg_t = neg_w;
-        }
-        if (neg_t) {
-            const uint64_t a = sub(u, t), b = add(u, t);
-            u = a;
-            v = b;
-        } else {
-            const uint64_t a = add(u, t), b = sub(u, t);
-            u = a;
-            v = b;
-        }
-    }
+    // w = +-2^S with S = e mod 96; from S = 32 on the negative -(v 2^S) is the
+    // cheaper form, which flips the sign once more.
+    constexpr int e = E % 192, S = e % 96;
+    constexpr bool neg_t = (e >= 96) != (S >= 32);
+    uint64_t t;
+    if constexpr (S >= 32) t = shl_mod_neg<S>(v);
+    else t = shl_mod<S>(v);
+    const uint64_t d = sub(u, t);
+    uint64_t a;
+    if constexpr (neg_t ? CV : CU) a = add(u, t);
+    else a = add_lazy(u, t);
+    u = neg_t ? d : a;
+    v = neg_t ? a : d;
 }
 
 // Field element of a signed 64-bit integer y with |y| < 2^63: y, or y + p
@@ -215,22 +237,47 @@ __host__ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// Which positions must be canonical after the stage of span LEN of an
+// N = 2^LOG point dit_pow2 with root 2^EW, so that the positions in `need` are
+// canonical after its last stage: backwards through the later stages, u of a
+// pair for either output, v of a pair whose twiddle is trivial.
+constexpr uint64_t dit_need_after(int log, int ew, int len, uint64_t need) {
+    const int n = 1 << log;
+    for (int l = n; l > len; l >>= 1) {
+        const int half = l / 2;
+        uint64_t before = 0;
+        for (int s = 0; s < n; s += l)
+            for (int k = 0; k < half; ++k) {
+                if (((need >> (s + k)) | (need >> (s + k + half))) & 1) before |= uint64_t{1} << (s + k);
+                if ((ew * k * (n / l)) % 96 == 0) before |= uint64_t{1} << (s + k + half);
+            }
+        need = before;
+    }
+    return need;
+}
+
+constexpr uint64_t DIT_ALL = ~uint64_t{0};
+
 // In-place radix-2 DIT DFT of length N = 2^LOG with root 2^EW on v[], which
-// holds the input in bit-reversed order; output in natural order.
-template <int LOG, int EW, int LEN = 2>
+// holds the input in bit-reversed order; output in natural order.  Inputs are
+// canonical; the outputs in NEED are canonical, the others any u64 (enough for
+// a value that a multiplication follows).
+template <int LOG, int EW, int LEN = 2, uint64_t NEED = DIT_ALL>
 __host__ __device__ __forceinline__ void dit_pow2(uint64_t* v) {
     if constexpr (LEN <= (1 << LOG)) {
         constexpr int N = 1 << LOG;
         constexpr int HALF = LEN / 2;
+        constexpr uint64_t C = dit_need_after(LOG, EW, LEN, NEED);
         static_for<0, N / LEN>([&](auto g) {
             constexpr int start = decltype(g)::value * LEN;
             static_for<0, HALF>([&](auto kk) {
                 constexpr int k = decltype(kk)::value;
                 // w_LEN^k = w_N^(k N/LEN) = 2^(EW k N/LEN)
-                bfly_pow2<EW * k * (N / LEN)>(v[start + k], v[start + k + HALF]);
+                bfly_pow2<EW * k * (N / LEN), ((C >> (start + k)) & 1) != 0, ((C >> (start + k + HALF)) & 1) != 0>(
+                    v[start + k], v[start + k + HALF]);
             });
         });
-        dit_pow2<LOG, EW, LEN * 2>(v);
+        dit_pow2<LOG, EW, LEN * 2, NEED>(v);
     }
 }
 
@@ -250,25 +297,28 @@ constexpr uint64_t dit_mask_next(uint64_t m, int len, int n) {
 // butterfly whose second input is known zero is the copy (u, u), one whose
 // inputs are both known zero is skipped, so a zero tail of the input costs no
 // arithmetic in the stages it reaches.  Runs the stages of spans LEN, 2 LEN,
-// ... below STOP (all of them by default).
-template <int LOG, int EW, uint64_t MASK, int LEN = 2, int STOP = (2 << LOG)>
+// ... below STOP (all of them by default); NEED as in dit_pow2, after the last
+// stage of the whole DFT.
+template <int LOG, int EW, uint64_t MASK, int LEN = 2, int STOP = (2 << LOG), uint64_t NEED = DIT_ALL>
 __host__ __device__ __forceinline__ void dit_pow2_sparse(uint64_t* v) {
     if constexpr (LEN <= (1 << LOG) && LEN < STOP) {
         constexpr int N = 1 << LOG;
         constexpr int HALF = LEN / 2;
+        constexpr uint64_t C = dit_need_after(LOG, EW, LEN, NEED);
         static_for<0, N / LEN>([&](auto g) {
             constexpr int start = decltype(g)::value * LEN;
             static_for<0, HALF>([&](auto kk) {
                 constexpr int k = decltype(kk)::value;
                 constexpr bool nz_u = (MASK >> (start + k)) & 1, nz_v = (MASK >> (start + k + HALF)) & 1;
                 if constexpr (nz_v) {
-                    bfly_pow2<EW * k * (N / LEN)>(v[start + k], v[start + k + HALF]);
+                    bfly_pow2<EW * k * (N / LEN), ((C >> (start + k)) & 1) != 0, ((C >> (start + k + HALF)) & 1) != 0>(
+                        v[start + k], v[start + k + HALF]);
                 } else if constexpr (nz_u) {
                     v[start + k + HALF] = v[start + k];
                 }
             });
         });
-        dit_pow2_sparse<LOG, EW, dit_mask_next(MASK, LEN, N), LEN * 2, STOP>(v);
+        dit_pow2_sparse<LOG, EW, dit_mask_next(MASK, LEN, N), LEN * 2, STOP, NEED>(v);
     }
 }
 

@@ -42,12 +42,27 @@ constexpr auto bfly_table(std::integer_sequence<int, E...>) {
     return std::array<B, sizeof...(E)>{+[](uint64_t* u, uint64_t* v) { gl::bfly_pow2<E>(*u, *v); }...};
 }
 const auto kBfly = bfly_table(std::make_integer_sequence<int, 192>{});
+template <int... E>
+constexpr auto bfly_lazy_table(std::integer_sequence<int, E...>) {
+    using B = void (*)(uint64_t*, uint64_t*);
+    return std::array<B, sizeof...(E)>{+[](uint64_t* u, uint64_t* v) { gl::bfly_pow2<E, false, false>(*u, *v); }...};
+}
+const auto kBflyLazy = bfly_lazy_table(std::make_integer_sequence<int, 192>{});
 }  // namespace
 
 extern "C" __attribute__((visibility("default"))) uint64_t glc_mul_pow2(uint64_t x, int e) { return kPow2[e](x); }
 extern "C" __attribute__((visibility("default"))) uint64_t glc_i16_mul_w128(int32_t x, int k) { return kW128[k](x); }
 extern "C" __attribute__((visibility("default"))) uint64_t glc_i16_mul_pow2(int32_t x, int e) { return kI16[e](x); }
 extern "C" __attribute__((visibility("default"))) void glc_bfly(uint64_t* u, uint64_t* v, int e) { kBfly[e](u, v); }
+// The same without canonical results (any u64 u; any u64 v where e mod 96 != 0).
+extern "C" __attribute__((visibility("default"))) void glc_bfly_lazy(uint64_t* u, uint64_t* v, int e) { kBflyLazy[e](u, v); }
+extern "C" __attribute__((visibility("default"))) uint64_t glc_add_lazy(uint64_t a, uint64_t b) { return gl::add_lazy(a, b); }
+extern "C" __attribute__((visibility("default"))) uint64_t glc_fold96_lazy(uint64_t lo, uint32_t hi) { return gl::fold96_lazy(lo, hi); }
+// The 16- and 32-point DFTs on bit-reversed canonical inputs, only output 0 canonical.
+extern "C" __attribute__((visibility("default"))) void glc_dft_lazy(uint64_t* v, int log) {
+    if (log == 5) gl::dit_pow2<5, gl::E_W32, 2, 1>(v);
+    else gl::dit_pow2<4, 2 * gl::E_W32, 2, 1>(v);
+}
 extern "C" __attribute__((visibility("default"))) uint64_t glc_mul32x4(uint64_t a, uint64_t b) { return gl::mul32x4(a, b); }
 extern "C" __attribute__((visibility("default"))) uint64_t glc_add(uint64_t a, uint64_t b) { return gl::add(a, b); }
 extern "C" __attribute__((visibility("default"))) uint64_t glc_sub(uint64_t a, uint64_t b) { return gl::sub(a, b); }
@@ -168,7 +183,7 @@ int n15_emulate(const uint64_t* fwd, const Src& src, size_t rows, size_t blocks,
                     else x1_read<1>(lds, v[t].data(), r.j1b, r.k3b);
                 }
             }
-            for (int t = 0; t < THREADS; ++t) gl::dit_pow2<5, gl::E_W32>(v[t].data());
+            for (int t = 0; t < THREADS; ++t) gl::dit_pow2<5, gl::E_W32, 2, 1>(v[t].data());
             for (int rd = 0; rd < 2; ++rd) {
                 poison();
                 for (int t = 0; t < THREADS; ++t) {
@@ -265,13 +280,13 @@ int rr_emulate(const uint64_t* fwd, const uint64_t* in, size_t stride, size_t le
                         for (int j3 = 8; j3 < 32; ++j3) tail = tail || v[t][gl::bitrev_c(j3, 5)] != 0;
                     ++(tail ? g_rr_waves_full : g_rr_waves_copy);
                     for (int t = w0; t < w0 + 64; ++t) {
-                        if (tail) gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(32), 2, 8>(v[t].data());
-                        else gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(8), 2, 8>(v[t].data());
-                        gl::dit_pow2<5, gl::E_W32, 8>(v[t].data());
+                        if (tail) gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(32), 2, 8, 1>(v[t].data());
+                        else gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(8), 2, 8, 1>(v[t].data());
+                        gl::dit_pow2<5, gl::E_W32, 8, 1>(v[t].data());
                     }
                 }
             } else {
-                for (int t = 0; t < S::THREADS; ++t) gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ)>(v[t].data());
+                for (int t = 0; t < S::THREADS; ++t) gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ), 2, 64, 1>(v[t].data());
             }
             for (int rd = 0; rd < 2; ++rd) {
                 poison();
@@ -289,7 +304,7 @@ int rr_emulate(const uint64_t* fwd, const uint64_t* in, size_t stride, size_t le
                     else x1_read<B, 1>(lds, v[t].data(), r.j1b, r.k3b);
                 }
             }
-            for (int t = 0; t < S::THREADS; ++t) gl::dit_pow2<5, gl::E_W32>(v[t].data());
+            for (int t = 0; t < S::THREADS; ++t) gl::dit_pow2<5, gl::E_W32, 2, 1>(v[t].data());
             for (int rd = 0; rd < 2; ++rd) {
                 poison();
                 for (int t = 0; t < S::THREADS; ++t) {

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(THREADS) void ntt15_rows(Src src, size_t rows, cons
             else x1_read<1>(lds, v, q.j1b, q.k3b);
         }
         __syncthreads();
-        gl::dit_pow2<5, gl::E_W32>(v);
+        gl::dit_pow2<5, gl::E_W32, 2, 1>(v);  // only B[0] meets no twiddle before stage C
         gl::static_for<0, 2>([&](auto rr) {
             constexpr int rd = decltype(rr)::value;
             {

@@ -205,7 +205,8 @@ __host__ __device__ __forceinline__ void stage_a(uint64_t* v, const Src& s, cons
         constexpr int j3 = decltype(j_)::value;
         v[gl::bitrev_c(j3, 5)] = s.template value<j3>(raw[j3]);
     });
-    gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ)>(v);
+    // only A[0] meets no twiddle before stage B
+    gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ), 2, 64, 1>(v);
 }
 
 // A distinct empty asm statement at both ends of each half's code: the two

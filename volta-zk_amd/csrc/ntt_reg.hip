@@ -96,8 +96,9 @@ __device__ __forceinline__ void park(uint64_t* s, const uint64_t* v, uint32_t pc
     });
 }
 
-// Step 2's head: the B values of (pc, ka), DFT'd over jb (natural order over kb).
-template <int LB>
+// Step 2's head: the B values of (pc, ka), DFT'd over jb (natural order over kb);
+// the outputs in NEED are canonical.
+template <int LB, uint64_t NEED>
 __device__ __forceinline__ void unpark(const uint64_t* s, uint64_t* v, uint32_t pc, uint32_t ka, uint32_t PW,
                                        uint32_t pitch) {
     constexpr int B = 1 << LB;
@@ -105,7 +106,7 @@ __device__ __forceinline__ void unpark(const uint64_t* s, uint64_t* v, uint32_t 
         constexpr int jb = decltype(jb_)::value;
         v[gl::bitrev_c(jb, LB)] = s[pc + PW * jb + ka * pitch];
     });
-    gl::dit_pow2<LB, ew_log<LB>()>(v);
+    gl::dit_pow2<LB, ew_log<LB>(), 2, NEED>(v);
 }
 
 // Inputs of the gather pass.  Row `row` of a batch, element idx < n,
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
             const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
             v[gl::bitrev_c(ja, LA)] = src.finish(idx, raw[ja]);
         });
-        gl::dit_pow2_sparse<LA, ew_log<LA>(), prefix_mask(NZ, LA)>(v);
+        gl::dit_pow2_sparse<LA, ew_log<LA>(), prefix_mask(NZ, LA), 2, (2 << LA), 1>(v);  // park() twiddles all but v[0]
         park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
     }
     __syncthreads();
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
         const uint32_t ka = job & (A - 1), pc = job >> LA;
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, t = PL == 2 ? (pc >> 1) : pc;
         uint64_t v[B];
-        unpark<LB>(s, v, pc, ka, PW, pitch);
+        unpark<LB, 0>(s, v, pc, ka, PW, pitch);  // the next pass multiplies every element
         const uint64_t orow =
             rot ? gather_row((nat0 + t + rot) & lmask, d, mid_bits) : row0 + (static_cast<uint64_t>(t) << mid_bits);
         const uint64_t out0 = (orow << RB) + ka;
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, 
                 v[gl::bitrev_c(ja, LA)] = r;
             });
         }
-        gl::dit_pow2<LA, ew_log<LA>()>(v);
+        gl::dit_pow2<LA, ew_log<LA>(), 2, 1>(v);  // park() twiddles all but v[0]
         park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
     }
     __syncthreads();
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, 
         const uint32_t pc = job & (PW - 1), ka = job >> pwb;
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, c = PL == 2 ? (pc >> 1) : pc;
         uint64_t v[B];
-        unpark<LB>(s, v, pc, ka, PW, pitch);
+        unpark<LB, gl::DIT_ALL>(s, v, pc, ka, PW, pitch);
         gl::static_for<0, B>([&](auto kb_) {
             constexpr int kb = decltype(kb_)::value;
             a[PL * (base + ((static_cast<uint64_t>(ka) + A * kb) << lb) + c) + plane] = v[kb];

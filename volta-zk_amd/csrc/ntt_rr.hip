@@ -61,12 +61,12 @@ __global__ __launch_bounds__(Shape<B>::THREADS, Shape<B>::WAVES_PER_SIMD) void r
             uint64_t tail = 0;
             gl::static_for<8, 32>([&](auto j_) { tail |= v[gl::bitrev_c(decltype(j_)::value, 5)]; });
             if (__builtin_amdgcn_ballot_w64(tail != 0) != 0)
-                gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(32), 2, 8>(v);
+                gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(32), 2, 8, 1>(v);
             else
-                gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(8), 2, 8>(v);
-            gl::dit_pow2<5, gl::E_W32, 8>(v);
+                gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(8), 2, 8, 1>(v);
+            gl::dit_pow2<5, gl::E_W32, 8, 1>(v);
         } else {
-            gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ)>(v);
+            gl::dit_pow2_sparse<5, gl::E_W32, prefix_mask(NZ), 2, 64, 1>(v);
         }
         __builtin_amdgcn_sched_barrier(0);
         {
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(Shape<B>::THREADS, Shape<B>::WAVES_PER_SIMD) void r
             else x1_read<B, 1>(lds, v, q.j1b, q.k3b);
         }
         __syncthreads();
-        gl::dit_pow2<5, gl::E_W32>(v);
+        gl::dit_pow2<5, gl::E_W32, 2, 1>(v);  // only B[0] meets no twiddle before stage C
         gl::static_for<0, 2>([&](auto rr_) {
             constexpr int rd = decltype(rr_)::value;
             {
