@@ -1,0 +1,38 @@
+"""The Merkle levels (subtrees of up to ten levels per workgroup, joins by one
+lane or by a quad of lanes) and the chunk runs of the column hash, bit-exact
+against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+P = 0xFFFF_FFFF_0000_0001
+
+
+def tree_of(backend, m):
+    rows, cols = m.shape
+    buf = backend.upload_device(m.reshape(-1))
+    tree = backend.hash_fp_tree_device(buf, rows, cols)
+    got = backend.download_device(tree.storage).reshape(2 * cols - 1, 32)
+    backend.free_device_merkle_tree(tree)
+    backend.free_device(buf)
+    return got
+
+
+# one workgroup's sizes on both sides of the quad switch (256), of its limit
+# (1,024), then one and two rounds of subtrees
+@pytest.mark.parametrize("bits", [0, 1, 2, 5, 7, 8, 9, 10, 11, 12, 16, 18, 19])
+def test_tree_levels(backend, oracle, bits):
+    m = np.random.Generator(np.random.PCG64(bits)).integers(0, P, size=(3, 1 << bits), dtype=np.uint64)
+    leaves = oracle.hash_fp_columns(m, *m.shape)
+    assert (tree_of(backend, m) == oracle.merkle_tree(leaves).reshape(-1, 32)).all()
+
+
+# runs of one, two and four chunks per thread, with a short last run and a
+# short last chunk (the columns decide which: 64 columns to a wave)
+@pytest.mark.parametrize("rows,bits", [(129, 6), (700, 8), (1300, 10), (300, 18), (140, 19)])
+def test_chunk_runs(backend, oracle, rows, bits):
+    m = np.random.Generator(np.random.PCG64(rows)).integers(0, P, size=(rows, 1 << bits), dtype=np.uint64)
+    got = tree_of(backend, m)
+    leaves = oracle.hash_fp_columns(m, rows, 1 << bits)
+    assert (got[:1 << bits] == leaves.reshape(-1, 32)).all()

@@ -22,7 +22,8 @@
 //   merge_pass: one thread per (column, run of 16 values) folds them with an
 //     eager join stack in LDS, repeated until one value per column is left;
 //     the column's last join carries the ROOT flag.
-//   merkle_level / merkle_top: the pair hashes of the Merkle tree.
+//   merkle_subtrees: the pair hashes of the Merkle tree, up to ten levels of a
+//     subtree per workgroup.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -160,8 +161,8 @@ constexpr size_t CHUNK_WORDS = 128; // u64 words per 1024-byte chunk
 // and 2+3 pair up, then the pairs; a short last group of 3 joins (0+1)+2.
 // Writes the group's chaining value to out[(g cols + col) 8 ..], or with
 // root set (one group per column) the column's leaf hash to out[col 8 ..].
-// OFF32: a row of the matrix spans less than 4 GiB, so a lane's element is
-// addressed as the uniform row pointer plus a 32-bit byte offset.
+// OFF32: the rows of a block span less than 4 GiB, so a lane's element is
+// addressed as the block's uniform pointer plus a 32-bit byte offset.
 template <int W, bool OFF32>
 __global__ __launch_bounds__(LANES, 6) void column_groups(const uint64_t* __restrict__ m, size_t rows, size_t cols,
                                                        size_t chunks, size_t group, int root,
@@ -181,40 +182,50 @@ __global__ __launch_bounds__(LANES, 6) void column_groups(const uint64_t* __rest
     const size_t last_words = words - (c_end - 1) * CHUNK_WORDS;
     const size_t total = (n_local - 1) * 16 + (min(CHUNK_WORDS, last_words) + 7) / 8;
 
-    auto element = [&](size_t row, int part) -> const uint64_t* {
-        const uint64_t* rowp = m + row * row_stride;
-        if constexpr (OFF32)
-            return reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(rowp) + lane_bytes) + part;
-        else
-            return rowp + col * W + part;
-    };
+    // Blocks load in stream order, RB rows each.  OFF32: a buffer resource at
+    // the block's first row, the lane's column as the 32-bit offset and the
+    // row's distance as a scalar one, so a block costs no vector address
+    // arithmetic and its addresses eight scalars (as 64-bit row pointers they
+    // spilled scalars into vector lanes, 133 moves per pair of blocks; 1,531
+    // rows x 4,096 columns 51 -> 49 us, the largest within 0.5%: the
+    // compressions themselves bound those).
+    constexpr int RB = 8 / W;
+    const size_t row0 = c_begin * CHUNK_WORDS / W;
+    const uint64_t* blk = m + row0 * row_stride;
     auto load_block = [&](size_t k, uint32_t* mw) {
         const size_t w0 = (c_begin * 16 + k) * 8;
         if (w0 + 8 <= words) {
-            if constexpr (W == 1) {
+            if constexpr (OFF32) {
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                    const_cast<uint64_t*>(blk), static_cast<short>(0), -1, 0x00020000);
+                const uint32_t stride = static_cast<uint32_t>(row_stride * sizeof(uint64_t));
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint64_t x = *element(w0 + i, 0);
-                    mw[2 * i] = static_cast<uint32_t>(x);
-                    mw[2 * i + 1] = static_cast<uint32_t>(x >> 32);
+                for (int i = 0; i < RB; ++i) {
+                    if constexpr (W == 1) {
+                        const auto x = __builtin_amdgcn_raw_buffer_load_b64(r, lane_bytes, i * stride, 0);
+                        mw[2 * i] = x[0], mw[2 * i + 1] = x[1];
+                    } else {  // one 16-byte (c0, c1) load per row
+                        const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, lane_bytes, i * stride, 0);
+                        mw[4 * i] = x[0], mw[4 * i + 1] = x[1], mw[4 * i + 2] = x[2], mw[4 * i + 3] = x[3];
+                    }
                 }
             } else {
-                using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {  // one 16-byte (c0, c1) load per row
-                    const u32x4 x = *reinterpret_cast<const u32x4*>(element(w0 / 2 + i, 0));
-                    mw[4 * i] = x.x, mw[4 * i + 1] = x.y, mw[4 * i + 2] = x.z, mw[4 * i + 3] = x.w;
+                for (int i = 0; i < 8; ++i) {
+                    const uint64_t x = blk[(i / W) * row_stride + col * W + i % W];
+                    mw[2 * i] = static_cast<uint32_t>(x);
+                    mw[2 * i + 1] = static_cast<uint32_t>(x >> 32);
                 }
             }
         } else {  // the column's last, partial block: zero past the end
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const size_t w = w0 + i;
-                const uint64_t x = w < words ? *element(w / W, static_cast<int>(w % W)) : 0;
+                const uint64_t x = w0 + i < words ? blk[(i / W) * row_stride + col * W + i % W] : 0;
                 mw[2 * i] = static_cast<uint32_t>(x);
                 mw[2 * i + 1] = static_cast<uint32_t>(x >> 32);
             }
         }
+        blk += RB * row_stride;
     };
 
     const uint32_t top = root ? PARENT | ROOT : PARENT;  // flags of the group's last join
@@ -376,53 +387,129 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_final(const uint32_t* __r
 
 constexpr uint32_t PAIR_FLAGS = CHUNK_START | CHUNK_END | ROOT;  // blake3 of a 64-byte message
 
-// parents[i] = blake3(child[2i] || child[2i+1])
-__global__ __launch_bounds__(256) void merkle_level(const uint32_t* __restrict__ child, uint32_t* __restrict__ parent,
-                                                    size_t parents) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= parents) return;
-    uint32_t l[8], r[8], p[8];
-    load_hash(l, child + 2 * i * 8);
-    load_hash(r, child + (2 * i + 1) * 8);
-    join(p, l, r, PAIR_FLAGS);
-    store_hash(parent + i * 8, p);
+// One compression split over a quad of lanes: lane i holds column i of the
+// 4 x 4 state, the diagonal half-rounds rotate rows 1..3 across the quad (DPP),
+// and the lane's 28 message words come from LDS at byte offsets that depend on
+// i only.  A join is then about 270 instructions deep instead of 690, at 1.5
+// times the total work: for the upper tree levels, whose few joins leave the
+// machine idle and whose depth is the time.
+struct Quad {
+    uint32_t off[7][4];      // byte offsets of the lane's words: two per half-round
+    uint32_t iva, ivb, len;  // IV[i], IV[4 + i] and the block length of state word 14
+    bool flag_lane;          // lane 3 holds the flags (state word 15)
+};
+
+__device__ __forceinline__ Quad make_quad(uint32_t i) {
+    Quad q;
+    gl::static_for<0, 28>([&](auto z_) {
+        constexpr int r = decltype(z_)::value / 4, j = decltype(z_)::value % 4, pos = j < 2 ? j : 6 + j;
+        constexpr uint32_t c = (4u * SCHED[r][pos]) | (4u * SCHED[r][pos + 2]) << 8 | (4u * SCHED[r][pos + 4]) << 16 |
+                               (4u * SCHED[r][pos + 6]) << 24;
+        q.off[r][j] = (c >> (8 * i)) & 255u;
+    });
+    q.iva = i == 0 ? IV[0] : i == 1 ? IV[1] : i == 2 ? IV[2] : IV[3];
+    q.ivb = i == 0 ? IV[4] : i == 1 ? IV[5] : i == 2 ? IV[6] : IV[7];
+    q.len = i == 2 ? 64u : 0u;
+    q.flag_lane = i == 3;
+    return q;
 }
 
-constexpr int TOP_THREADS = 512;
-constexpr size_t TOP_MAX = 2 * TOP_THREADS;  // nodes a single workgroup finishes
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_perm(uint32_t x) {
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xF, 0xF, true));
+}
 
-// The last levels in one workgroup: level (at tree + off 8, len <= TOP_MAX
-// nodes) up to the root, staged through LDS and written level by level.
-__global__ __launch_bounds__(TOP_THREADS) void merkle_top(uint32_t* __restrict__ tree, size_t off, int len) {
-    __shared__ uint32_t cur[TOP_MAX][9];
+// Words i and 4 + i of compress(IV, the 16 words at msg, 0, 64, flags), for
+// lane i of a quad whose four lanes are active and share msg (LDS).
+__device__ __forceinline__ void quad_join(const Quad& q, const uint32_t* msg, uint32_t flags, uint32_t* lo,
+                                          uint32_t* hi) {
+    uint32_t w[7][4];
+    gl::static_for<0, 28>([&](auto z_) {
+        constexpr int r = decltype(z_)::value / 4, j = decltype(z_)::value % 4;
+        w[r][j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(msg) + q.off[r][j]);
+    });
+    uint32_t a = q.iva, b = q.ivb, c = q.iva, d = q.flag_lane ? flags : q.len;
+    constexpr int NEXT = 0x39, OPPOSITE = 0x4E, PREV = 0x93;  // lane i reads lane i + 1, i + 2, i + 3 (mod 4)
+    gl::static_for<0, 7>([&](auto r_) {
+        constexpr int r = decltype(r_)::value;
+        g(a, b, c, d, w[r][0], w[r][1]);
+        b = quad_perm<NEXT>(b);
+        c = quad_perm<OPPOSITE>(c);
+        d = quad_perm<PREV>(d);
+        g(a, b, c, d, w[r][2], w[r][3]);
+        b = quad_perm<PREV>(b);
+        c = quad_perm<OPPOSITE>(c);
+        d = quad_perm<NEXT>(d);
+    });
+    *lo = a ^ c;
+    *hi = b ^ d;
+}
+
+constexpr int TREE_THREADS = 512;
+constexpr int TREE_QUADS = TREE_THREADS / 4;
+constexpr size_t TREE_MAX = 1024;  // nodes one workgroup takes at most
+constexpr size_t TREE_SPAN = 256;  // nodes per workgroup while the level has more than TREE_MAX
+constexpr int MSG_PITCH = 17;      // words per pair of children: 16 and a pad against bank conflicts
+
+// Workgroup b builds the subtree over nodes [b span, (b + 1) span) of a level
+// (len nodes at tree + off 8; span a power of two, 2 <= span <= TREE_MAX,
+// dividing len) up to its root, staging levels through two LDS buffers and
+// writing each to its place in the tree.  A level of more than TREE_QUADS
+// joins takes one lane per join, the others a quad of lanes.  Column hash and
+// tree of 24 rows x 256 columns 19.7 -> 14.5 us, 7 x 131,072 48 -> 28 us, against
+// one launch per level down to 1,024 nodes and one lane per join throughout.
+__global__ __launch_bounds__(TREE_THREADS) void merkle_subtrees(uint32_t* __restrict__ tree, size_t off, size_t len,
+                                                               int span) {
+    __shared__ uint32_t even[TREE_MAX / 2 * MSG_PITCH], odd[TREE_MAX / 4 * MSG_PITCH];
     const int t = threadIdx.x;
-    for (int i = t; i < len; i += TOP_THREADS) {
+    const uint32_t i = t & 3;
+    size_t base = static_cast<size_t>(blockIdx.x) * span;
+    // node n sits in pair n / 2, half n & 1
+    for (int n = t; n < span; n += TREE_THREADS) {
         uint32_t h[8];
-        load_hash(h, tree + (off + i) * 8);
+        load_hash(h, tree + (off + base + n) * 8);
+        uint32_t* dst = even + (n >> 1) * MSG_PITCH + 8 * (n & 1);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) cur[i][k] = h[k];
+        for (int k = 0; k < 8; ++k) dst[k] = h[k];
     }
+    const Quad quad = make_quad(i);
+    uint32_t *cur = even, *up = odd;
     __syncthreads();
-    while (len > 1) {
-        const int parents = len / 2;  // len is a power of two
-        uint32_t p[8];
-        if (t < parents) {
-            uint32_t l[8], r[8];
+    for (int parents = span / 2; parents > 0; parents /= 2) {
+        off += len;
+        len /= 2;
+        base /= 2;
+        if (parents > TREE_QUADS) {
+            if (t < parents) {
+                uint32_t m[16], cv[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                l[k] = cur[2 * t][k];
-                r[k] = cur[2 * t + 1][k];
+                for (int k = 0; k < 16; ++k) m[k] = cur[t * MSG_PITCH + k];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) cv[k] = IV[k];
+                compress(cv, m, 0, 64, PAIR_FLAGS);
+                store_hash(tree + (off + base + t) * 8, cv);
+                uint32_t* dst = up + (t >> 1) * MSG_PITCH + 8 * (t & 1);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) dst[k] = cv[k];
             }
-            join(p, l, r, PAIR_FLAGS);
-            store_hash(tree + (off + len + t) * 8, p);
+        } else {
+            const int n = t >> 2;
+            if (n < parents) {
+                uint32_t lo, hi;
+                quad_join(quad, cur + n * MSG_PITCH, PAIR_FLAGS, &lo, &hi);
+                uint32_t* dst = up + (n >> 1) * MSG_PITCH + 8 * (n & 1) + i;
+                dst[0] = lo;
+                dst[4] = hi;
+                uint32_t* node = tree + (off + base + n) * 8 + i;
+                node[0] = lo;
+                node[4] = hi;
+            }
         }
         __syncthreads();
-        if (t < parents)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) cur[t][k] = p[k];
-        __syncthreads();
-        off += len;
-        len = parents;
+        uint32_t* const s = cur;
+        cur = up;
+        up = s;
     }
 }
 
@@ -453,11 +540,29 @@ __global__ __launch_bounds__(256) void merkle_paths_kernel(const uint32_t* __res
 }  // namespace b3
 
 
+// Chunks per column_groups thread: the most (4, 2 or 1) that still gives every
+// SIMD its 6 waves, since longer runs leave fewer chaining values to store and
+// join; below that the time is the run's own length and short runs win.  The
+// whole tree with 4 / 2 / 1 chunks per thread, microseconds: 1,531 rows x 4,096
+// columns 129 / 82 / 61; 3,000 x 8,192 136 / 125 / 109; 8,192 x 8,192 222 / 217 /
+// 215; 8,192 x 16,384 385 / 380 / 380; above the line 2,080 x 131,072 705 / 716 /
+// 751; 24,576 x 32,768 1,967 / 2,004 / 2,116; 65,536 x 8,192 1,331 / 1,351 / 1,410.
+static size_t chunks_per_thread(const Context* c, size_t cols, size_t chunks) {
+    const size_t cus = c->cu_count > 0 ? static_cast<size_t>(c->cu_count) : 256;
+    const size_t full = cus * 4 * 6, waves = (cols + b3::LANES - 1) / b3::LANES;
+    for (size_t g : {size_t{4}, size_t{2}}) {
+        // half as long runs would exceed the launch grid's second dimension
+        const bool limit = (chunks + g / 2 - 1) / (g / 2) > 65535;
+        if (limit || waves * ((chunks + g - 1) / g) >= full) return std::min(g, chunks);
+    }
+    return 1;
+}
+
 int merkle_column_leaves(Context* c, const uint64_t* m, size_t rows, size_t cols, bool fp2, uint32_t* leaves) {
     const size_t w = fp2 ? 2 : 1;
     const size_t words = rows * w;
     const size_t chunks = (words + b3::CHUNK_WORDS - 1) / b3::CHUNK_WORDS;
-    const size_t group = std::min<size_t>(4, chunks);  // chunks per column_groups thread
+    const size_t group = chunks_per_thread(c, cols, chunks);
     size_t k = (chunks + group - 1) / group;           // values per column after column_groups
     if (k > 65535) return fail_msg(c, "Merkle column too long (more than 2^18 BLAKE3 chunks)");
     // workspace: column_groups' values, then each non-final merge pass's (16x fewer)
@@ -473,7 +578,7 @@ int merkle_column_leaves(Context* c, const uint64_t* m, size_t rows, size_t cols
     const dim3 grid(static_cast<unsigned>((cols + b3::LANES - 1) / b3::LANES), static_cast<unsigned>(k));
     const int is_root = k == 1 ? 1 : 0;
     uint32_t* gout = k == 1 ? leaves : buf;
-    const bool off32 = cols * w * sizeof(uint64_t) <= 0xFFFFFFFFull;
+    const bool off32 = cols <= 0xFFFFFFFFull / 64;  // a block is 64 bytes of every column
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(b3::LANES), 0, c->stream, m, rows, cols, chunks, group, is_root, gout);
     };
@@ -506,18 +611,15 @@ int merkle_column_leaves(Context* c, const uint64_t* m, size_t rows, size_t cols
 
 int merkle_tree_levels(Context* c, uint32_t* tree, size_t leaves) {
     size_t off = 0, len = leaves;
-    while (len > b3::TOP_MAX) {
-        const size_t parents = len / 2;
-        hipLaunchKernelGGL(b3::merkle_level, dim3(static_cast<unsigned>((parents + 255) / 256)), dim3(256), 0,
-                           c->stream, static_cast<const uint32_t*>(tree + off * 8), tree + (off + len) * 8, parents);
+    while (len > 1) {
+        const size_t span = len > b3::TREE_MAX ? b3::TREE_SPAN : len;
+        hipLaunchKernelGGL(b3::merkle_subtrees, dim3(static_cast<unsigned>(len / span)), dim3(b3::TREE_THREADS), 0,
+                           c->stream, tree, off, len, static_cast<int>(span));
         VMX_HIP(c, hipGetLastError());
-        off += len;
-        len = parents;
-    }
-    if (len > 1) {
-        hipLaunchKernelGGL(b3::merkle_top, dim3(1), dim3(b3::TOP_THREADS), 0, c->stream, tree, off,
-                           static_cast<int>(len));
-        VMX_HIP(c, hipGetLastError());
+        for (size_t n = span; n > 1; n /= 2) {
+            off += len;
+            len /= 2;
+        }
     }
     return 0;
 }
