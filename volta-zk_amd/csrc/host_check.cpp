@@ -248,9 +248,8 @@ extern "C" __attribute__((visibility("default"))) int glc_ntt15_msg(const uint64
 // all zero from 8 M on, in full otherwise; the waves of each kind are counted.
 namespace {
 long g_rr_waves_full = 0, g_rr_waves_copy = 0;
-template <int B, int NZ>
-int rr_emulate(const uint64_t* fwd, const uint64_t* in, size_t stride, size_t len, size_t rows, size_t blocks,
-               uint64_t* out) {
+template <int B, int NZ, class Src>
+int rr_emulate(const uint64_t* fwd, const Src& src, size_t rows, size_t blocks, uint64_t* out) {
     using namespace vmx::rr;
     using S = Shape<B>;
     constexpr int GUARD = 64;
@@ -272,7 +271,7 @@ int rr_emulate(const uint64_t* fwd, const uint64_t* in, size_t stride, size_t le
     for (size_t b = 0; b < blocks; ++b) {
         for (int t = 0; t < S::T2_WORDS; ++t) lds[S::T2_OFF + t] = tab[S::T1_WORDS + t];
         for (size_t row = b; row < rows; row += blocks) {
-            for (int t = 0; t < S::THREADS; ++t) load_row<B, NZ>(v[t].data(), in, stride, len, row, role<B>(t).m);
+            for (int t = 0; t < S::THREADS; ++t) load_row<B, NZ>(v[t].data(), src, row, role<B>(t).m);
             if constexpr (NZ == 32) {
                 for (int w0 = 0; w0 < S::THREADS; w0 += 64) {
                     bool tail = false;
@@ -335,9 +334,24 @@ int rr_dispatch(const uint64_t* fwd, const uint64_t* in, size_t stride, size_t l
                 uint64_t* out) {
     using S = vmx::rr::Shape<B>;
     if (len == 0 || len > size_t{S::N} || stride < len) return 1;
-    if (len <= size_t{8} * S::M) return rr_emulate<B, 8>(fwd, in, stride, len, rows, blocks, out);
-    if (len <= size_t{16} * S::M) return rr_emulate<B, 16>(fwd, in, stride, len, rows, blocks, out);
-    return rr_emulate<B, 32>(fwd, in, stride, len, rows, blocks, out);
+    const vmx::rr::SrcU64 s{in, stride, len};
+    if (len <= size_t{8} * S::M) return rr_emulate<B, 8>(fwd, s, rows, blocks, out);
+    if (len <= size_t{16} * S::M) return rr_emulate<B, 16>(fwd, s, rows, blocks, out);
+    return rr_emulate<B, 32>(fwd, s, rows, blocks, out);
+}
+
+// The kernels' choice for message rows (rr::msg_rows).
+template <int B>
+int rr_msg_dispatch(const uint64_t* fwd, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows,
+                    size_t blocks, uint64_t* out) {
+    using namespace vmx::rr;
+    constexpr size_t M = Shape<B>::M;
+    if (cols == 0 || cols + pad > size_t{Shape<B>::N}) return 1;
+    if (cols == 8 * M && pad == 0) return rr_emulate<B, 8>(fwd, SrcMsg<8>{w, pads, cols, pad}, rows, blocks, out);
+    if (cols == 8 * M && pad <= 2 * M) return rr_emulate<B, 10>(fwd, SrcMsg<8>{w, pads, cols, pad}, rows, blocks, out);
+    if (cols == 4 * M && pad <= 2 * M) return rr_emulate<B, 6>(fwd, SrcMsg<4>{w, pads, cols, pad}, rows, blocks, out);
+    if (cols + pad <= 16 * M) return rr_emulate<B, 16>(fwd, SrcMsg<0>{w, pads, cols, pad}, rows, blocks, out);
+    return rr_emulate<B, 32>(fwd, SrcMsg<0>{w, pads, cols, pad}, rows, blocks, out);
 }
 }  // namespace
 
@@ -359,4 +373,11 @@ extern "C" __attribute__((visibility("default"))) int glc_ntt14r_u64(const uint6
                                                                      size_t stride, size_t len, size_t rows,
                                                                      size_t blocks, uint64_t* out) {
     return rr_dispatch<4>(fwd, in, stride, len, rows, blocks, out);
+}
+extern "C" __attribute__((visibility("default"))) int glc_ntt_rr_msg(const uint64_t* fwd, const int16_t* w,
+                                                                     const uint64_t* pads, size_t cols, size_t pad,
+                                                                     size_t bits, size_t rows, size_t blocks,
+                                                                     uint64_t* out) {
+    return bits == 13 ? rr_msg_dispatch<3>(fwd, w, pads, cols, pad, rows, blocks, out)
+                      : rr_msg_dispatch<4>(fwd, w, pads, cols, pad, rows, blocks, out);
 }

@@ -44,6 +44,9 @@ int ntt13r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
                     TwiddleSet* t);
 int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, size_t n, uint64_t* out,
                     TwiddleSet* t);
+// The same for message rows lift(w) || pads || 0 of either size.
+int ntt_rr_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
+                    uint64_t* out, TwiddleSet* t);
 // The n = 2^13 tables of ntt13r inside the encode's device table (built on
 // first use; null on error), and their builder.
 const uint64_t* enc13_rr_table(Context* c, TwiddleSet* t);

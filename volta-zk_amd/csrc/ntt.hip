@@ -191,6 +191,11 @@ int ntt_fp2_rows(Context* c, const uint64_t* in, size_t rows, size_t n, uint64_t
 
 int ntt_msg_i16_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t rows, size_t cols, size_t pad,
                      size_t n, uint64_t* out, TwiddleSet* t) {
+    // n = 2^13, 2^14 and (most shapes) 2^15: one pass over HBM
+    if (n == 8192 || n == 16384) {
+        const int rc = ntt_rr_msg_rows(c, w, pads, cols, pad, rows, n, out, t);
+        if (rc <= 0) return rc;
+    }
     if (n == 32768) {
         const int rc = ntt15_msg_rows(c, w, pads, cols, pad, rows, n, out, t);
         if (rc <= 0) return rc;

@@ -1,5 +1,5 @@
-// ntt_rr.hip -- one-pass forward NTT of u64 rows of 2^13 and 2^14 points held
-// in registers (the split, the roles and the exchanges are in ntt_rr.hpp).
+// ntt_rr.hip -- one-pass forward NTT of u64 and message rows of 2^13 and 2^14
+// points held in registers (the split, the roles and the exchanges are in ntt_rr.hpp).
 //
 // Persistent workgroups of 32 N1 threads (four per CU for 2^13, one for
 // 2^14; Shape::PER_CU), one row each at a time, without prefetch: the other
@@ -18,10 +18,9 @@ namespace rr {
 
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
-template <int B, int NZ>
+template <int B, int NZ, class Src>
 __global__ __launch_bounds__(Shape<B>::THREADS, Shape<B>::WAVES_PER_SIMD) void rows_kernel(
-    const uint64_t* __restrict__ in, size_t stride, size_t len, size_t rows, const uint64_t* __restrict__ tab,
-    uint64_t* __restrict__ out) {
+    Src src, size_t rows, const uint64_t* __restrict__ tab, uint64_t* __restrict__ out) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using S = Shape<B>;
     extern __shared__ uint64_t lds[];
@@ -50,7 +49,7 @@ __global__ __launch_bounds__(Shape<B>::THREADS, Shape<B>::WAVES_PER_SIMD) void r
     __builtin_amdgcn_s_setprio(1);
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         uint64_t v[32], tw[8];
-        load_row<B, NZ>(v, in, stride, len, row, here().m);
+        load_row<B, NZ>(v, src, row, here().m);
         if constexpr (NZ == 32) {
             // Rows the length does not bound (a buffer the caller may have
             // written through a device pointer) are often still zero from
@@ -136,20 +135,45 @@ __global__ void build_table(const uint64_t* __restrict__ fwd, uint64_t* __restri
     if (idx < Shape<B>::TABLE_WORDS) tab[idx] = table_word<B>(fwd, idx);
 }
 
-template <int B>
-int launch(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, const uint64_t* tab,
-           uint64_t* out) {
+template <int B, int NZ, class Src>
+int launch(Context* c, const Src& src, size_t rows, const uint64_t* tab, uint64_t* out) {
     using S = Shape<B>;
     const size_t cus = c->cu_count > 0 ? static_cast<size_t>(c->cu_count) : 256;
     const unsigned blocks = static_cast<unsigned>(std::min(rows, S::PER_CU * cus));
-    auto k = len <= size_t{8} * S::M ? rows_kernel<B, 8> : len <= size_t{16} * S::M ? rows_kernel<B, 16>
-                                                                                     : rows_kernel<B, 32>;
+    auto k = rows_kernel<B, NZ, Src>;
     if (S::LDS_BYTES > 65536)
         VMX_HIP(c, hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(S::LDS_BYTES)));
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(S::THREADS), S::LDS_BYTES, c->stream, in, stride, len, rows, tab, out);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(S::THREADS), S::LDS_BYTES, c->stream, src, rows, tab, out);
     VMX_HIP(c, hipGetLastError());
     return 0;
+}
+
+// The kernel whose stage A reads the fewest of its 32 inputs covering the row.
+template <int B>
+int u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, const uint64_t* tab,
+             uint64_t* out) {
+    constexpr size_t M = Shape<B>::M;
+    const SrcU64 s{in, stride, len};
+    if (len <= 8 * M) return launch<B, 8>(c, s, rows, tab, out);
+    if (len <= 16 * M) return launch<B, 16>(c, s, rows, tab, out);
+    return launch<B, 32>(c, s, rows, tab, out);
+}
+
+// Message rows: cols of 8 or 4 whole blocks of M (rates 1/4 and 1/8) with pads
+// of at most two blocks read each block from one source; other shapes read
+// both.  8,192 rows of 2^11 + 512 into 2^13: the whole commitment 722 -> 566 us
+// against the pass engine's two passes (446 us of kernels).
+template <int B>
+int msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows,
+             const uint64_t* tab, uint64_t* out) {
+    constexpr size_t M = Shape<B>::M;
+    const uint64_t* pp = pad ? pads : tab;  // a readable word when there are no pads
+    if (cols == 8 * M && pad == 0) return launch<B, 8>(c, SrcMsg<8>{w, pp, cols, pad}, rows, tab, out);
+    if (cols == 8 * M && pad <= 2 * M) return launch<B, 10>(c, SrcMsg<8>{w, pp, cols, pad}, rows, tab, out);
+    if (cols == 4 * M && pad <= 2 * M) return launch<B, 6>(c, SrcMsg<4>{w, pp, cols, pad}, rows, tab, out);
+    if (cols + pad <= 16 * M) return launch<B, 16>(c, SrcMsg<0>{w, pp, cols, pad}, rows, tab, out);
+    return launch<B, 32>(c, SrcMsg<0>{w, pp, cols, pad}, rows, tab, out);
 }
 
 int build14(Context* c, TwiddleSet* t) {
@@ -176,7 +200,7 @@ int ntt13r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
     if (rows == 0) return 0;
     const uint64_t* tab = enc13_rr_table(c, t);
     if (!tab) return -1;
-    return rr::launch<3>(c, in, stride, len, rows, tab, out);
+    return rr::u64_rows<3>(c, in, stride, len, rows, tab, out);
 }
 
 int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, size_t n, uint64_t* out,
@@ -185,7 +209,22 @@ int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
     if (!t->grid && c->coarse_active) return 1;
     if (rows == 0) return 0;
     if (ensure_grid_twiddles(c, t, size_t{rr::Shape<4>::TABLE_WORDS} * sizeof(uint64_t), rr::build14)) return -1;
-    return rr::launch<4>(c, in, stride, len, rows, t->grid, out);
+    return rr::u64_rows<4>(c, in, stride, len, rows, t->grid, out);
+}
+
+int ntt_rr_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
+                    uint64_t* out, TwiddleSet* t) {
+    const bool b3 = n == static_cast<size_t>(rr::Shape<3>::N), b4 = n == static_cast<size_t>(rr::Shape<4>::N);
+    if ((!b3 && !b4) || cols == 0 || cols + pad > n || !t->fwd) return 1;
+    if (!t->grid && c->coarse_active) return 1;
+    if (rows == 0) return 0;
+    if (b3) {
+        const uint64_t* tab = enc13_rr_table(c, t);
+        if (!tab) return -1;
+        return rr::msg_rows<3>(c, w, pads, cols, pad, rows, tab, out);
+    }
+    if (ensure_grid_twiddles(c, t, size_t{rr::Shape<4>::TABLE_WORDS} * sizeof(uint64_t), rr::build14)) return -1;
+    return rr::msg_rows<4>(c, w, pads, cols, pad, rows, t->grid, out);
 }
 
 }  // namespace vmx

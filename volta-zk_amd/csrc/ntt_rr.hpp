@@ -1,6 +1,6 @@
-// ntt_rr.hpp -- the phases of the one-pass forward NTT of u64 rows of
-// n = 32 x 32 x N1 points (N1 = 2^B: 2^13 for B = 3, 2^14 for B = 4) whose
-// elements may all be nonzero, as host/device functions of one thread, so
+// ntt_rr.hpp -- the phases of the one-pass forward NTT of rows of
+// n = 32 x 32 x N1 points (N1 = 2^B: 2^13 for B = 3, 2^14 for B = 4), u64 rows
+// whose elements may all be nonzero or message rows, as host/device functions of one thread, so
 // that a host build can run them thread by thread between the kernel's
 // barriers (host_check.cpp).
 //
@@ -130,25 +130,81 @@ struct Table1 {
 #endif
 };
 
-// Row `row` of x (stride elements apart, len u64 then zeros): element
-// m + 32 N1 j3 for j3 < NZ into slot bitrev5(j3), the rest zero.
-template <int B, int NZ>
-__host__ __device__ __forceinline__ void load_row(uint64_t* v, const uint64_t* x, size_t stride, size_t len,
-                                                  size_t row, int m) {
-    constexpr int M = Shape<B>::M;
-    gl::static_for<0, 32>([&](auto i_) { v[decltype(i_)::value] = 0; });
+// Sources of stage A's inputs: element m + M j3 of row `row`, zero past the
+// row's end.  On the device every read goes through a buffer resource that
+// spans exactly the row's part, so what lies past it reads as zero.
+// SrcU64: x + row stride, len u64 then zeros.
+struct SrcU64 {
+    const uint64_t* x;
+    size_t stride, len;
+    template <int M, int NZ>
+    __host__ __device__ __forceinline__ void load(uint64_t* v, size_t row, int m) const {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const auto r = rsrc(x + row * stride, len * 8);
+        const auto r = rsrc(x + row * stride, len * 8);
 #endif
-    gl::static_for<0, NZ>([&](auto j_) {
-        constexpr int j3 = decltype(j_)::value;
+        gl::static_for<0, NZ>([&](auto j_) {
+            constexpr int j3 = decltype(j_)::value;
 #if defined(__HIP_DEVICE_COMPILE__)
-        v[gl::bitrev_c(j3, 5)] = ld64(r, static_cast<uint32_t>(m) * 8u, j3 * (M * 8u));
+            v[gl::bitrev_c(j3, 5)] = ld64(r, static_cast<uint32_t>(m) * 8u, j3 * (M * 8u));
 #else
-        const size_t idx = static_cast<size_t>(m) + size_t{M} * j3;
-        v[gl::bitrev_c(j3, 5)] = idx < len ? x[row * stride + idx] : 0;
+            const size_t idx = static_cast<size_t>(m) + size_t{M} * j3;
+            v[gl::bitrev_c(j3, 5)] = idx < len ? x[row * stride + idx] : 0;
 #endif
-    });
+        });
+    }
+};
+
+// SrcMsg: lift(w) || pads || 0 (reference pcs_messages_kernel,
+// cuda/volta_cuda_backend.cu:2950-2958).  WB > 0: cols = WB M, so blocks j3 < WB
+// are weights and the others pads.  WB = 0: any cols; every block reads both
+// parts, of which at most one is not zero.  pads must point at a readable word
+// even when pad = 0.
+template <int WB>
+struct SrcMsg {
+    const int16_t* w;
+    const uint64_t* pads;
+    size_t cols, pad;
+    template <int M, int NZ>
+    __host__ __device__ __forceinline__ void load(uint64_t* v, size_t row, int m) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const auto rw = rsrc(w + row * cols, cols * 2), rp = rsrc(pads + row * pad, pad * 8);
+        uint32_t h[NZ];
+        uint64_t q[NZ];
+        gl::static_for<0, NZ>([&](auto j_) {
+            constexpr int j3 = decltype(j_)::value;
+            if constexpr (WB == 0 || j3 < WB)
+                h[j3] = __builtin_amdgcn_raw_buffer_load_b16(rw, static_cast<uint32_t>(m) * 2u, j3 * (M * 2u), 0);
+            if constexpr (WB == 0) {
+                const uint32_t idx = static_cast<uint32_t>(m) + M * j3, c = static_cast<uint32_t>(cols);
+                q[j3] = ld64(rp, idx >= c ? (idx - c) * 8u : 0x7FFFFFF8u, 0);
+            } else if constexpr (j3 >= WB) {
+                q[j3] = ld64(rp, static_cast<uint32_t>(m) * 8u, (j3 - WB) * (M * 8u));
+            }
+        });
+        __builtin_amdgcn_sched_barrier(0);  // all of the row's loads in flight before the first lift
+        gl::static_for<0, NZ>([&](auto j_) {
+            constexpr int j3 = decltype(j_)::value;
+            uint64_t x = 0;
+            if constexpr (WB == 0 || j3 < WB) x = gl::from_i16(static_cast<int16_t>(static_cast<uint16_t>(h[j3])));
+            if constexpr (WB == 0 || j3 >= WB) x |= q[j3];
+            v[gl::bitrev_c(j3, 5)] = x;
+        });
+#else
+        for (int j3 = 0; j3 < NZ; ++j3) {
+            const size_t idx = static_cast<size_t>(m) + size_t{M} * j3;
+            v[gl::bitrev_c(j3, 5)] = idx < cols         ? gl::from_i16(w[row * cols + idx])
+                                     : idx - cols < pad ? pads[row * pad + (idx - cols)]
+                                                        : 0;
+        }
+#endif
+    }
+};
+
+// Row `row`: element m + 32 N1 j3 for j3 < NZ into slot bitrev5(j3), the rest zero.
+template <int B, int NZ, class Src>
+__host__ __device__ __forceinline__ void load_row(uint64_t* v, const Src& src, size_t row, int m) {
+    gl::static_for<0, 32>([&](auto i_) { v[decltype(i_)::value] = 0; });
+    src.template load<Shape<B>::M, NZ>(v, row, m);
 }
 
 // A distinct empty asm statement at both ends of each half's code: the two
