@@ -1,7 +1,7 @@
 // ntt_rr.hip -- one-pass forward NTT of u64 and message rows of 2^13 and 2^14
 // points held in registers (the split, the roles and the exchanges are in ntt_rr.hpp).
 //
-// Persistent workgroups of 32 N1 threads (four per CU for 2^13, one for
+// Persistent workgroups of 32 N1 threads (four per CU for 2^13, two for
 // 2^14; Shape::PER_CU), one row each at a time, without prefetch: the other
 // workgroups on the CU run while one waits on its row's loads.  Each store
 // instruction writes two runs of 32 consecutive u64.

@@ -41,10 +41,11 @@ struct Shape {
     static constexpr int LOG_N = 10 + B;
     static constexpr int N = 1 << LOG_N;
     static constexpr int THREADS = 32 * N1;
-    // Workgroups per CU: four 4-wave workgroups at 128 VGPRs for 2^13; one
-    // 8-wave workgroup for 2^14, whose stage C (two 16-point DFTs per thread)
-    // takes 174 VGPRs (at 128 it spilled 61-80).
-    static constexpr int PER_CU = B == 3 ? 4 : 1;
+    // Workgroups per CU: four of 4 waves for 2^13, two of 8 waves for 2^14 (70 KiB of
+    // LDS each), both 4 waves per SIMD at 128 VGPRs.  2^14 rows of 2^12 inputs with
+    // two instead of one: 1,000 rows 86.8 -> 63.5 us, 16,384 rows 1,431 -> 975 us,
+    // up to 256 rows (one per CU either way) unchanged.
+    static constexpr int PER_CU = B == 3 ? 4 : 2;
     static constexpr int WAVES_PER_SIMD = PER_CU * THREADS / 256;
     static constexpr int P = 32 / N1;  // stage-C pairs per thread
     static constexpr int M = 32 * N1;  // stage-A rows m = j1 + N1 j2
