@@ -3,8 +3,8 @@
 // (ntt.hip: NttPlan::forward semantics, rust/volta-pcs/src/ntt.rs:34-70) and by
 // the X4 Fp2 transform (x4.hip, rust/volta-pcs/src/x4/ntt.rs:66-122).
 //
-// An n = 2^nb point transform, n = R_1 R_2 .. R_P with every R_p <= 2^8 (2^9 for
-// one-plane rows below 2^26, ntt_reg.hpp: pass_bits), runs in
+// An n = 2^nb point transform, n = R_1 R_2 .. R_P with every R_p <= 2^8 (2^9 below
+// 2^26 points, ntt_reg.hpp: pass_bits), runs in
 // P passes (decimation in time by the least significant input digit first):
 //   pass 1 ("gather"): row r = (i_1, .., i_(P-1)) (i_1 most significant) gets
 //     the R_P-point DFT of x[nat(r) + (n / R_P) j], j < R_P, with
@@ -39,6 +39,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "context.hpp"
 #include "gl64.hpp"
@@ -82,18 +83,59 @@ __device__ __forceinline__ void fill_park_twiddles(uint64_t* ptw, const uint64_t
         ptw[i] = inner_pow(inner, ((i >> LA) * (i & (A - 1))) << (GBITS - RB));
 }
 
-// Step 1's tail: v (natural order over ka after the A-point DFT) times
-// w_R^(jb ka), parked at (pc, jb, ka).
-template <int LA, int LB>
+// Step 1's tail: outputs ka in [K0, K0 + KN) of v (natural order over ka after the
+// A-point DFT) times w_R^(jb ka), parked at (pc, jb, ka - K0).
+template <int LA, int LB, int K0 = 0, int KN = 1 << LA>
 __device__ __forceinline__ void park(uint64_t* s, const uint64_t* v, uint32_t pc, uint32_t jb, uint32_t PW,
                                      uint32_t pitch, const uint64_t* ptw) {
     constexpr int A = 1 << LA;
-    s[pc + PW * jb] = v[0];
     const uint64_t* row = ptw + jb * A;
-    gl::static_for<1, A>([&](auto ka_) {
+    gl::static_for<K0, K0 + KN>([&](auto ka_) {
         constexpr int ka = decltype(ka_)::value;
-        s[pc + PW * jb + ka * pitch] = gl::mul32x4(v[ka], row[ka]);
+        s[pc + PW * jb + (ka - K0) * pitch] = ka ? gl::mul32x4(v[ka], row[ka]) : v[0];
     });
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// A span of device memory at a uniform address: an access is one 32-bit lane
+// offset plus a scalar one, so the 32 accesses of a radix-2^9 job hold one
+// address register instead of a pair each.
+struct Span {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Span(const uint64_t* p, uint64_t bytes)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t*>(p), static_cast<short>(0),
+                                              static_cast<int>(bytes), 0x00020000)) {}
+    __device__ __forceinline__ uint64_t at(uint32_t voff, uint32_t soff) const {
+        const auto t = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+        return static_cast<uint64_t>(t[0]) | (static_cast<uint64_t>(t[1]) << 32);
+    }
+    __device__ __forceinline__ void put(uint32_t voff, uint32_t soff, uint64_t x) const {
+        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+        __builtin_amdgcn_raw_buffer_store_b64(v2u{static_cast<uint32_t>(x), static_cast<uint32_t>(x >> 32)}, r, voff,
+                                              soff, 0);
+    }
+};
+#else
+struct Span {  // the host pass only parses the kernels
+    __device__ Span(const uint64_t*, uint64_t) {}
+    __device__ uint64_t at(uint32_t, uint32_t) const { return 0; }
+    __device__ void put(uint32_t, uint32_t, uint64_t) const {}
+};
+#endif
+
+// Radix 2^9 (A = 32): a workgroup's 16 x 16 step-1 jobs are one per thread, so the
+// 32 outputs stay in registers and go through LDS in two rounds of 16 (step 2's
+// 512 jobs, 256 per round).  Half the LDS and at most 128 registers: four
+// workgroups per CU instead of two.  2^17 x 2,048 rows 1,976 -> 1,812 us, 2^18 x
+// 1,024 2,164 -> 1,948, 2^25 x 4 1,519 -> 1,453; and two planes can take the
+// radix, which saves them a pass at 2^17, 2^18 and 2^25 (plan()).
+template <int LA>
+constexpr bool two_rounds() {
+    return LA == 5;
+}
+template <int LA>
+constexpr int parked() {  // outputs per step-1 job in LDS at a time
+    return two_rounds<LA>() ? 16 : 1 << LA;
 }
 
 // Step 2's head: the B values of (pc, ka), DFT'd over jb (natural order over kb);
@@ -208,7 +250,7 @@ __device__ __forceinline__ uint64_t gather_row(uint64_t L, const Digits& d, int 
 // 128-byte line per run instead of two (only the wrap to L = 0 in the last
 // tile straddles).  The rows still cover 0 .. n / R - 1 once.
 template <int LA, int LB, int PL, int NZ, class Src>
-__global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restrict__ y, int nb, int qb, Digits d,
+__global__ __launch_bounds__(THREADS, two_rounds<LA>() ? 4 : 1) void gather_reg(Src src, uint64_t* __restrict__ y, int nb, int qb, Digits d,
                                                       const uint64_t* inner) {
     constexpr int A = 1 << LA, B = 1 << LB, RB = LA + LB;
     static_assert(NZ >= 1 && NZ <= A, "step 1 reads between 1 and A inputs");
@@ -222,7 +264,7 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
     // pc + ka pitch, then meet distinct banks in every 32-lane group when
     // pitch = 32 / A (mod 32) words; step 1's writes are contiguous per ka.
     const uint32_t pitch = PW * B + 32 / A;
-    uint64_t* ptw = s + A * pitch;  // the inner twiddles follow the tile
+    uint64_t* ptw = s + parked<LA>() * pitch;  // the inner twiddles follow the tile
     fill_park_twiddles<LA, LB>(ptw, inner);
     __syncthreads();
     uint64_t nat0, row0;
@@ -235,8 +277,7 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
     // (B-point DFTs, stores), so co-resident workgroups interleave their
     // phases (measured: C4 +6%, p15 +3%, X4 2^24 +3%, C5 and p17 within 2%).
     __builtin_amdgcn_s_setprio(1);
-    for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
-        const uint32_t pc = job & (PW - 1), jb = job >> pwb;
+    auto step1 = [&](uint32_t pc, uint32_t jb, uint64_t* v) {
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, t = PL == 2 ? (pc >> 1) : pc;
         const uint64_t L = (nat0 + t + rot) & lmask;
         typename Src::Raw raw[NZ];
@@ -245,7 +286,6 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
             const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
             raw[ja] = src.fetch(row, idx, plane, PL);
         });
-        uint64_t v[A];
         gl::static_for<0, A>([&](auto i_) { v[decltype(i_)::value] = 0; });
         gl::static_for<0, NZ>([&](auto ja_) {
             constexpr int ja = decltype(ja_)::value;
@@ -253,15 +293,12 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
             v[gl::bitrev_c(ja, LA)] = src.finish(idx, raw[ja]);
         });
         gl::dit_pow2_sparse<LA, ew_log<LA>(), prefix_mask(NZ, LA), 2, (2 << LA), 1>(v);  // park() twiddles all but v[0]
-        park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
-    }
-    __syncthreads();
-    __builtin_amdgcn_s_setprio(0);
-    for (uint32_t job = threadIdx.x; job < (PW << LA); job += THREADS) {
-        const uint32_t ka = job & (A - 1), pc = job >> LA;
+    };
+    // outputs ka + A kb of (pc, ka), parked at ka - k0
+    auto step2 = [&](uint32_t pc, uint32_t ka, uint32_t k0) {
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, t = PL == 2 ? (pc >> 1) : pc;
         uint64_t v[B];
-        unpark<LB, 0>(s, v, pc, ka, PW, pitch);  // the next pass multiplies every element
+        unpark<LB, 0>(s, v, pc, ka - k0, PW, pitch);  // the next pass multiplies every element
         const uint64_t orow =
             rot ? gather_row((nat0 + t + rot) & lmask, d, mid_bits) : row0 + (static_cast<uint64_t>(t) << mid_bits);
         const uint64_t out0 = (orow << RB) + ka;
@@ -269,6 +306,29 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
             constexpr int kb = decltype(kb_)::value;
             y[PL * (out0 + A * kb) + plane] = v[kb];
         });
+    };
+    if constexpr (two_rounds<LA>()) {
+        const uint32_t job = threadIdx.x;
+        uint64_t v[A];
+        step1(job & 15, job >> 4, v);
+        park<LA, LB, 0, 16>(s, v, job & 15, job >> 4, PW, pitch, ptw);
+        __syncthreads();
+        step2(job >> 4, job & 15, 0);
+        __syncthreads();
+        park<LA, LB, 16, 16>(s, v, job & 15, job >> 4, PW, pitch, ptw);
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
+        step2(job >> 4, 16 + (job & 15), 16);
+    } else {
+        for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
+            const uint32_t pc = job & (PW - 1), jb = job >> pwb;
+            uint64_t v[A];
+            step1(pc, jb, v);
+            park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
+        }
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
+        for (uint32_t job = threadIdx.x; job < (PW << LA); job += THREADS) step2(job >> LA, job & (A - 1), 0);
     }
 }
 
@@ -290,7 +350,7 @@ __global__ __launch_bounds__(THREADS) void gather_reg(Src src, uint64_t* __restr
 // row.  Keeping all rows of a tile on one XCD, so that the slice is read once,
 // measured 2.7% slower on C5.
 template <int LA, int LB, int PL, int MODE, bool TBL>
-__global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, int lb, int cb, const uint64_t* inner,
+__global__ __launch_bounds__(THREADS, two_rounds<LA>() ? 4 : 1) void col_reg(uint64_t* a, int nb, int hb, int lb, int cb, const uint64_t* inner,
                                                    const uint64_t* split, int split_h, const uint64_t* ctab,
                                                    uint64_t scale, int rows_inner) {
     static_assert(PL == 2 || MODE == ROOT_BASE, "one-plane transforms stop at 2^31 points");
@@ -307,7 +367,7 @@ __global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, 
     const int pwb = cb + (PL - 1);
     const uint32_t PW = 1u << pwb;
     const uint32_t pitch = PW * (B + 1);
-    uint64_t* ptw = s + A * pitch;  // the inner twiddles follow the tile
+    uint64_t* ptw = s + parked<LA>() * pitch;  // the inner twiddles follow the tile
     fill_park_twiddles<LA, LB>(ptw, inner);
     __syncthreads();
     const uint64_t lblocks = (uint64_t{1} << lb) >> cb;
@@ -319,12 +379,28 @@ __global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, 
     // (B-point DFTs, stores), so co-resident workgroups interleave their
     // phases (measured: C4 +6%, p15 +3%, X4 2^24 +3%, C5 and p17 within 2%).
     __builtin_amdgcn_s_setprio(1);
-    for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
-        const uint32_t pc = job & (PW - 1), jb = job >> pwb;
+    auto step1 = [&](uint32_t pc, uint32_t jb, uint64_t* v) {
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, c = PL == 2 ? (pc >> 1) : pc;
         const uint64_t l = l0 + c;
-        uint64_t v[A];
-        if constexpr (TBL) {
+        if constexpr (two_rounds<LA>() && TBL) {
+            // as below, through buffer resources, the table 8 words at a time
+            const uint64_t bytes = (uint64_t{8} << RB) << lb;
+            const Span xs(a + PL * base, PL * bytes), ts(ctab, bytes);
+            const uint32_t off = (((jb << lb) + c) * PL + plane) * 8, step = (8u * B) << lb;
+            const uint32_t toff = ((jb << lb) + static_cast<uint32_t>(l)) * 8;
+            uint64_t xv[A], tv[8];
+            gl::static_for<0, A>(
+                [&](auto ja_) { xv[decltype(ja_)::value] = xs.at(off, decltype(ja_)::value * PL * step); });
+            gl::static_for<0, A / 8>([&](auto q_) {
+                constexpr int q = 8 * decltype(q_)::value;
+                gl::static_for<0, 8>([&](auto i_) { tv[decltype(i_)::value] = ts.at(toff, (q + decltype(i_)::value) * step); });
+                __builtin_amdgcn_sched_barrier(0);
+                gl::static_for<0, 8>([&](auto i_) {
+                    constexpr int i = decltype(i_)::value;
+                    v[gl::bitrev_c(q + i, LA)] = gl::mul32x4(xv[q + i], tv[i]);
+                });
+            });
+        } else if constexpr (TBL) {
             // the job's A inputs and A table words, all in flight, then A products
             uint64_t xv[A], tv[A];
             gl::static_for<0, A>([&](auto ja_) {
@@ -411,19 +487,45 @@ __global__ __launch_bounds__(THREADS) void col_reg(uint64_t* a, int nb, int hb, 
             });
         }
         gl::dit_pow2<LA, ew_log<LA>(), 2, 1>(v);  // park() twiddles all but v[0]
-        park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
-    }
-    __syncthreads();
-    __builtin_amdgcn_s_setprio(0);
-    for (uint32_t job = threadIdx.x; job < (PW << LA); job += THREADS) {
-        const uint32_t pc = job & (PW - 1), ka = job >> pwb;
+    };
+    // outputs ka + A kb of (pc, ka), parked at ka - k0
+    auto step2 = [&](uint32_t pc, uint32_t ka, uint32_t k0) {
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, c = PL == 2 ? (pc >> 1) : pc;
         uint64_t v[B];
-        unpark<LB, gl::DIT_ALL>(s, v, pc, ka, PW, pitch);
-        gl::static_for<0, B>([&](auto kb_) {
-            constexpr int kb = decltype(kb_)::value;
-            a[PL * (base + ((static_cast<uint64_t>(ka) + A * kb) << lb) + c) + plane] = v[kb];
-        });
+        unpark<LB, gl::DIT_ALL>(s, v, pc, ka - k0, PW, pitch);
+        if constexpr (two_rounds<LA>()) {
+            const Span ys(a + PL * base, (uint64_t{PL * 8} << RB) << lb);
+            const uint32_t off = (((ka << lb) + c) * PL + plane) * 8, step = (PL * 8u * A) << lb;
+            gl::static_for<0, B>([&](auto kb_) { ys.put(off, decltype(kb_)::value * step, v[decltype(kb_)::value]); });
+        } else {
+            gl::static_for<0, B>([&](auto kb_) {
+                constexpr int kb = decltype(kb_)::value;
+                a[PL * (base + ((static_cast<uint64_t>(ka) + A * kb) << lb) + c) + plane] = v[kb];
+            });
+        }
+    };
+    if constexpr (two_rounds<LA>()) {
+        const uint32_t pc = threadIdx.x & 15, q = threadIdx.x >> 4;
+        uint64_t v[A];
+        step1(pc, q, v);
+        park<LA, LB, 0, 16>(s, v, pc, q, PW, pitch, ptw);
+        __syncthreads();
+        step2(pc, q, 0);
+        __syncthreads();
+        park<LA, LB, 16, 16>(s, v, pc, q, PW, pitch, ptw);
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
+        step2(pc, 16 + q, 16);
+    } else {
+        for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
+            const uint32_t pc = job & (PW - 1), jb = job >> pwb;
+            uint64_t v[A];
+            step1(pc, jb, v);
+            park<LA, LB>(s, v, pc, jb, PW, pitch, ptw);
+        }
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
+        for (uint32_t job = threadIdx.x; job < (PW << LA); job += THREADS) step2(job & (PW - 1), job >> pwb, 0);
     }
 }
 
@@ -477,7 +579,7 @@ constexpr uint64_t BIG_TABLE_ROWS = 16;
 
 template <int LA, int LB, int PL>
 ColFn col_for(int mode, bool tbl) {
-    if constexpr (PL == 2) {
+    if constexpr (PL == 2 && LA < 5) {  // radix 2^9 stops below 2^26 points
         if (mode == nreg::ROOT_NEG32) return nreg::col_reg<LA, LB, PL, nreg::ROOT_NEG32, false>;
         if (mode == nreg::ROOT_IMAG33) return nreg::col_reg<LA, LB, PL, nreg::ROOT_IMAG33, false>;
     }
@@ -517,39 +619,39 @@ bool kernels_for(int rb, int mode, uint64_t nza, bool tbl, GatherFn<Src>* g, Col
         case 6: *g = gather_for<3, 3, PL, Src>(nza); *col = col_for<3, 3, PL>(mode, tbl); break;
         case 7: *g = gather_for<4, 3, PL, Src>(nza); *col = col_for<4, 3, PL>(mode, tbl); break;
         case 8: *g = gather_for<4, 4, PL, Src>(nza); *col = col_for<4, 4, PL>(mode, tbl); break;
-        case 9:
-            if constexpr (PL == 1) {
-                *g = gather_for<5, 4, PL, Src>(nza);
-                *col = col_for<5, 4, PL>(mode, tbl);
-                break;
-            }
-            return false;
+        case 9: *g = gather_for<5, 4, PL, Src>(nza); *col = col_for<5, 4, PL>(mode, tbl); break;
         default: return false;
     }
     return *col != nullptr;
 }
 
 // Pass radices: the fewest passes of at most 2^pass_bits, as even as possible.
-int plan(int nb, int planes, int* r) {
-    const int pb = nreg::pass_bits(nb, planes);
+// Two planes take radix 2^9 only in batches of at least 2^21 elements (`big`), whose
+// tiles give every CU work: 97 transforms of 2^17 257 -> 169 us, 8 of 2^18 54 -> 45,
+// one of 2^25 939 -> 665, but one of 2^17 13.9 -> 19.6 and one of 2^18 16.5 -> 27.7.
+int plan(int nb, int planes, bool big, int* r) {
+    const int pb = planes == 1 || big ? nreg::pass_bits(nb) : nreg::PASS_BITS;
     const int passes = (nb + pb - 1) / pb;
     if (nb < nreg::MIN_BITS || passes > nreg::MAX_PASSES) return 0;
     for (int p = 0; p < passes; ++p) r[p] = nb / passes + (p < nb % passes ? 1 : 0);
+    // Two planes (X4 encodes with a zero tail): the one radix 2^9 of 2^17 or 2^25
+    // points goes to the gather, which reads only the inputs before the tail.
+    if (planes == 2 && r[0] == 9) std::swap(r[0], r[passes - 1]);
     return passes;
 }
 
-// LDS bytes of a column tile: 2^pwb (coordinate, column) pairs x A x (B + 1)
-// words, then the R = A B inner twiddles.
+// LDS bytes of a column tile: 2^pwb (coordinate, column) pairs x A (two_rounds: 16)
+// x (B + 1) words, then the R = A B inner twiddles.
 size_t tile_lds(int rb, int pwb) {
-    const size_t A = size_t{1} << ((rb + 1) / 2), B = size_t{1} << (rb / 2);
-    return ((size_t{1} << pwb) * A * (B + 1) + A * B) * sizeof(uint64_t);
+    const size_t A = size_t{1} << ((rb + 1) / 2), B = size_t{1} << (rb / 2), K = std::min<size_t>(A, 16);
+    return ((size_t{1} << pwb) * K * (B + 1) + A * B) * sizeof(uint64_t);
 }
 
-// LDS bytes of a gather tile: A rows of 2^pwb B words, each padded by 32 / A,
+// LDS bytes of a gather tile: A (two_rounds: 16) rows of 2^pwb B words, each padded by 32 / A,
 // then the R = A B inner twiddles.
 size_t gather_lds(int rb, int pwb) {
-    const size_t A = size_t{1} << ((rb + 1) / 2), B = size_t{1} << (rb / 2);
-    return (((size_t{1} << pwb) * B) * A + 32 + A * B) * sizeof(uint64_t);
+    const size_t A = size_t{1} << ((rb + 1) / 2), B = size_t{1} << (rb / 2), K = std::min<size_t>(A, 16);
+    return (((size_t{1} << pwb) * B) * K + 32 + A * B) * sizeof(uint64_t);
 }
 
 template <class K>
@@ -566,7 +668,7 @@ bool reg_ntt_covers(uint64_t n) {
     int r[nreg::MAX_PASSES];
     int nb = 0;
     while ((uint64_t{1} << nb) < n) ++nb;
-    return (uint64_t{1} << nb) == n && plan(nb, 1, r) > 0;
+    return (uint64_t{1} << nb) == n && plan(nb, 1, false, r) > 0;
 }
 
 int derive_reg_tables(Context* c, TwiddleSet* t) {
@@ -623,7 +725,7 @@ static int col_table_for(Context* c, const RegTables& tb, int hb, int rb, int lb
 template <int PL, class Src, class Shift>
 int run_passes(Context* c, const RegTables& tb, Src src, Shift shift, uint64_t* out, uint64_t rows, int nb) {
     int r[nreg::MAX_PASSES] = {};
-    const int passes = plan(nb, PL, r);
+    const int passes = plan(nb, PL, (rows << nb) >= (uint64_t{1} << 21), r);
     if (passes == 0) return fail_msg(c, "NTT size outside the pass engine's range");
     // A scaled source (the inverse transform's n^-1) hands its scale to the
     // last column pass when that pass builds its pre-twiddles as a progression
@@ -669,7 +771,7 @@ int run_passes(Context* c, const RegTables& tb, Src src, Shift shift, uint64_t* 
             const int la = (rb + 1) / 2;
             const uint64_t nza = (s0.extent(uint64_t{1} << nb) + (uint64_t{1} << (nb - la)) - 1) >> (nb - la);
             if (!kernels_for<PL, Src>(rb, nreg::root_mode(nb), nza, false, &g, &col) || blocks > 0x7FFFFFFFull ||
-                lds > 160 * 1024)
+                lds > 160 * 1024 || (rb == 9 && qb + PL - 1 != 4))
                 return fail_msg(c, "NTT pass exceeds its launch limits");
             if (allow_lds(c, g, lds)) return -1;
             hipLaunchKernelGGL(g, dim3(static_cast<unsigned>(blocks), cnt), dim3(nreg::THREADS), lds, c->stream, s0, y,
@@ -690,7 +792,7 @@ int run_passes(Context* c, const RegTables& tb, Src src, Shift shift, uint64_t* 
             if (p == 0 && last_scale != 1 && ctab != nullptr)
                 return fail_msg(c, "inverse NTT scale handed to a column pass that reads a table");
             if (!kernels_for<PL, Src>(rb, nreg::root_mode(nb), 0, ctab != nullptr, &g, &col) ||
-                blocks > 0x7FFFFFFFull || lds > 160 * 1024)
+                blocks > 0x7FFFFFFFull || lds > 160 * 1024 || (rb == 9 && cb + PL - 1 != 4))
                 return fail_msg(c, "NTT pass exceeds its launch limits");
             if (allow_lds(c, col, lds)) return -1;
             const uint64_t pass_scale = p == 0 && ctab == nullptr ? last_scale : uint64_t{1};

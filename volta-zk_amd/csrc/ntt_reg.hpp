@@ -33,12 +33,11 @@ __host__ __device__ constexpr int run_bits(int nb, int planes) {
     return (nb >= 26 ? 4 : 3) + (planes == 1 ? 1 : 0);
 }
 
-// Largest radix of a pass for elements of `planes` u64: 2^9 for one-plane
-// rows below 2^26 points, whose radix-2^9 tiles stay at 70 KB of LDS (two per
-// CU); that saves a pass at 2^17, 2^18 and 2^25 (measured: 2^17 rows 4.4 ms
-// against 5.4 ms in three passes).  2^8 otherwise: a radix-2^9 tile of Fp2 or
-// of 32 adjacent rows needs 139 KB, one per CU, and ran 1.8x slower.
-__host__ __device__ constexpr int pass_bits(int nb, int planes) { return planes == 1 && nb < 26 ? 9 : PASS_BITS; }
+// Largest radix of a pass: 2^9 below 2^26 points, where a tile is 16 words wide
+// and its two LDS rounds (ntt_reg.hip: two_rounds) keep four workgroups on a CU;
+// that saves a pass at 2^17, 2^18 and 2^25 (two planes: of large batches, plan()).
+// 2^8 from 2^26 on, whose tiles are 32 words wide.
+__host__ __device__ constexpr int pass_bits(int nb) { return nb < 26 ? 9 : PASS_BITS; }
 
 // Tile index of this workgroup.  Workgroups are dispatched round-robin over
 // the 8 XCDs (blockIdx.x mod 8); with XCD_SWIZZLE the tiles an XCD runs back to
