@@ -178,7 +178,8 @@ enum WorkspaceSlot : int {
     WS_PARTIALS = 4,  // combination partial sums
     WS_AUX2 = 5,      // combination coefficient sums
     WS_HASH = 6,      // Merkle column-group chaining values
-    WS_COUNT = 7,
+    WS_FLAGS = 7,     // rejected-draw flags of ChaCha8 rows (zero between calls)
+    WS_COUNT = 8,
 };
 
 struct TimingRecord {

@@ -772,7 +772,17 @@ int gather_columns(Context* c, const uint64_t* m, const uint32_t* idx, uint64_t*
 // rejection (probability 2^-32 per draw) only shifts later places, and may
 // take one more round.  Draw m goes to out[r * stride + m]; the lanes of a
 // round write one contiguous run.
+// Nearly every round keeps all its draws: a lane's eight then go out as four
+// 16-byte stores without the scan (rows whose start allows it).
+// 8,192 rows of 512: 27.1 -> 16.3 us.
 constexpr int CHACHA_WAVES = 4;  // rows per 256-thread workgroup
+
+// The eight draws of a block to o (16-byte aligned).
+__device__ __forceinline__ void store_draws(uint64_t* o, const uint64_t* v) {
+    using u64x2 = uint64_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) reinterpret_cast<u64x2*>(o)[i] = u64x2{v[2 * i], v[2 * i + 1]};
+}
 
 __global__ __launch_bounds__(64 * CHACHA_WAVES) void chacha8_rows_kernel(chacha8::Key key, uint64_t base_domain,
                                                                          size_t rows, size_t draws, size_t stride,
@@ -791,6 +801,12 @@ __global__ __launch_bounds__(64 * CHACHA_WAVES) void chacha8_rows_kernel(chacha8
             for (int i = 0; i < 8; ++i) {
                 v[i] = static_cast<uint64_t>(w[2 * i]) | (static_cast<uint64_t>(w[2 * i + 1]) << 32);
                 kept += v[i] < chacha8::P ? 1 : 0;
+            }
+            if (done + 512 <= draws && (reinterpret_cast<uintptr_t>(o + done) & 15) == 0 &&
+                __builtin_amdgcn_ballot_w64(kept != 8) == 0) {
+                store_draws(o + done + 8 * lane, v);
+                done += 512;
+                continue;
             }
             int incl = kept;  // inclusive scan over the lanes
 #pragma unroll
@@ -812,21 +828,27 @@ __global__ __launch_bounds__(64 * CHACHA_WAVES) void chacha8_rows_kernel(chacha8
     }
 }
 
-// Few long rows (an opening's mask rows: claims + 1 rows of tens of
-// thousands of draws) would leave most of the GPU idle with one wave per row
-// and serialise a hundred rounds.  Here a workgroup of CHACHA_WIDE waves fills
-// one row: a round takes 64 CHACHA_WIDE consecutive blocks (wave w, lane t:
-// block k0 + 64 w + t), each wave scans its lanes' kept counts, and the waves'
-// totals (in LDS) place each wave's run after those of the waves before it --
-// the same places as the one-wave kernel, in 1/CHACHA_WIDE of the rounds.
+// Few long rows (an opening's mask rows: claims + 1 rows of tens of thousands of
+// draws) would leave most of the GPU idle with one wave per row.  They are
+// written by chacha8_spread_kernel as if no draw were rejected, one block per
+// thread over the whole GPU, and a row that does meet a rejection (probability
+// draws 2^-32) is flagged and written again, in order, by
+// chacha8_rows_wide_kernel: a workgroup of CHACHA_WIDE waves takes 64 CHACHA_WIDE
+// consecutive blocks per round (wave w, lane t: block k0 + 64 w + t), each wave
+// scans its lanes' kept counts, and the waves' totals (in LDS) place each wave's
+// run after those of the waves before it -- the same places as the one-wave
+// kernel, in 1/CHACHA_WIDE of the rounds.  Without flags it writes every row.
+// 7 rows of 66,560 draws: 78 us in order, 7.2 + 3.2 us spread.
 constexpr int CHACHA_WIDE = 16;
 
 __global__ __launch_bounds__(64 * CHACHA_WIDE) void chacha8_rows_wide_kernel(chacha8::Key key, uint64_t base_domain,
                                                                              size_t rows, size_t draws, size_t stride,
-                                                                             size_t zero_from, uint64_t* out) {
+                                                                             size_t zero_from, uint64_t* out,
+                                                                             uint32_t* flags) {
     __shared__ int wave_total[CHACHA_WIDE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (size_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        if (flags && flags[r] == 0) continue;  // uniform over the workgroup
         uint64_t* o = out + r * stride;
         size_t done = 0;  // kept draws so far (uniform over the workgroup)
         for (uint64_t k0 = 0; done < draws; k0 += 64 * CHACHA_WIDE) {
@@ -866,21 +888,71 @@ __global__ __launch_bounds__(64 * CHACHA_WIDE) void chacha8_rows_wide_kernel(cha
             __syncthreads();  // wave_total is rewritten by the next round
         }
         for (size_t z = zero_from + threadIdx.x; z < stride; z += 64 * CHACHA_WIDE) o[z] = 0;
+        // every thread read the flag before the rounds' barriers: clear for the next call
+        if (flags && threadIdx.x == 0) flags[r] = 0;
     }
 }
 
-// Rows of `draws` kept values at `stride` words, zero from zero_from: one wave
-// per row, or a workgroup per row for few long rows.
+constexpr int CHACHA_SPREAD = 256;
+
+__global__ __launch_bounds__(CHACHA_SPREAD) void chacha8_spread_kernel(chacha8::Key key, uint64_t base_domain,
+                                                                       size_t draws, size_t stride, size_t zero_from,
+                                                                       uint64_t* out, uint32_t* flags) {
+    const size_t r = blockIdx.y, k = static_cast<size_t>(blockIdx.x) * CHACHA_SPREAD + threadIdx.x;
+    uint64_t* o = out + r * stride;
+    if (8 * k < draws) {
+        uint32_t w[16];
+        chacha8::block(key, base_domain + r, k, w);
+        uint64_t v[8];
+        bool rejected = false;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] = static_cast<uint64_t>(w[2 * i]) | (static_cast<uint64_t>(w[2 * i + 1]) << 32);
+            rejected |= v[i] >= chacha8::P && 8 * k + i < draws;
+        }
+        if (8 * k + 8 <= draws && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
+            store_draws(o + 8 * k, v);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (8 * k + i < draws) o[8 * k + i] = v[i];
+        }
+        if (rejected) atomicOr(&flags[r], 1u);
+    }
+    for (size_t z = zero_from + k; z < stride; z += static_cast<size_t>(gridDim.x) * CHACHA_SPREAD) o[z] = 0;
+}
+
+constexpr size_t CHACHA_LONG_ROWS = 1024;  // most rows of the two kernels above
+
+// Rows of `draws` kept values at `stride` words, zero from zero_from: one wave per
+// row, or for few long rows the spread kernel and the ordered one behind its flags
+// (zero between calls: cleared when allocated and by the ordered kernel).  Inside a
+// coarse timing scope, where workspaces may not grow, missing flags leave the
+// ordered kernel alone.
 static int chacha8_rows(Context* c, const uint8_t seed[32], uint64_t base_domain, size_t rows, size_t draws,
                         size_t stride, size_t zero_from, uint64_t* out) {
     const chacha8::Key key = chacha8::key_from_seed(seed);
-    if (rows <= 1024 && draws >= 8192)
+    if (rows <= CHACHA_LONG_ROWS && draws >= 8192) {
+        constexpr size_t flag_bytes = CHACHA_LONG_ROWS * sizeof(uint32_t);
+        if (c->ws[WS_FLAGS].capacity < flag_bytes && !c->coarse_active) {
+            if (ensure_ws(c, WS_FLAGS, flag_bytes) || zero_bytes(c, c->ws[WS_FLAGS].ptr, flag_bytes)) return -1;
+        }
+        uint32_t* flags = ws<uint32_t>(c, WS_FLAGS);
+        if (flags) {
+            const size_t blocks = (draws + 8 * CHACHA_SPREAD - 1) / (8 * CHACHA_SPREAD);
+            hipLaunchKernelGGL(chacha8_spread_kernel,
+                               dim3(static_cast<unsigned>(std::min<size_t>(blocks, 0x7FFFFFFF)), static_cast<unsigned>(rows)),
+                               dim3(CHACHA_SPREAD), 0, c->stream, key, base_domain, draws, stride, zero_from, out,
+                               flags);
+            VMX_HIP(c, hipGetLastError());
+        }
         hipLaunchKernelGGL(chacha8_rows_wide_kernel, dim3(static_cast<unsigned>(rows)), dim3(64 * CHACHA_WIDE), 0,
-                           c->stream, key, base_domain, rows, draws, stride, zero_from, out);
-    else
+                           c->stream, key, base_domain, rows, draws, stride, zero_from, out, flags);
+    } else {
         hipLaunchKernelGGL(chacha8_rows_kernel, dim3(grid_for(rows, CHACHA_WAVES, size_t{1} << 20)),
                            dim3(64 * CHACHA_WAVES), 0, c->stream, key, base_domain, rows, draws, stride, zero_from,
                            out);
+    }
     VMX_HIP(c, hipGetLastError());
     return 0;
 }
@@ -1019,6 +1091,7 @@ __global__ __launch_bounds__(256) void eq_rows_kernel(const Fp2* __restrict__ po
 
 constexpr int DOT_THREADS = 1024;  // 16 waves per row: a claim's mask row is 2^13..2^17 long
 constexpr int DOT_UNROLL = 4;      // products whose loads are in flight together
+constexpr size_t DOT_PART = size_t{DOT_THREADS} * DOT_UNROLL;  // least elements of a part
 
 __device__ __forceinline__ Fp2 fp2_shfl_xor(Fp2 x, int m) {
     const uint64_t c0 = __shfl_xor(x.c0, m), c1 = __shfl_xor(x.c1, m);
@@ -1030,15 +1103,17 @@ __device__ __forceinline__ Fp2 fp2_shfl_xor(Fp2 x, int m) {
 // wave and one LDS step across the four waves.
 __global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __restrict__ a, size_t a_stride,
                                                                    const Fp2* __restrict__ b, size_t b_stride,
-                                                                   Fp2* __restrict__ out, size_t rows, size_t len) {
+                                                                   Fp2* __restrict__ out, size_t rows, size_t len,
+                                                                   size_t part_len) {
     __shared__ Fp2 part[DOT_THREADS / 64];
     const int t = threadIdx.x;
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         Fp2 acc{0, 0};
         const Fp2* ar = a + row * a_stride;
         const Fp2* br = b + row * b_stride;
-        size_t j = t;
-        for (; j + (DOT_UNROLL - 1) * DOT_THREADS < len; j += DOT_UNROLL * DOT_THREADS) {
+        size_t j = blockIdx.y * part_len + t;
+        const size_t end = min(len, (blockIdx.y + 1) * part_len);
+        for (; j + (DOT_UNROLL - 1) * DOT_THREADS < end; j += DOT_UNROLL * DOT_THREADS) {
             Fp2 x[DOT_UNROLL], y[DOT_UNROLL];
 #pragma unroll
             for (int u = 0; u < DOT_UNROLL; ++u) {
@@ -1048,7 +1123,7 @@ __global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __
 #pragma unroll
             for (int u = 0; u < DOT_UNROLL; ++u) acc = gl::fp2_add(acc, gl::fp2_mul(x[u], y[u]));
         }
-        for (; j < len; j += DOT_THREADS) acc = gl::fp2_add(acc, gl::fp2_mul(ar[j], br[j]));
+        for (; j < end; j += DOT_THREADS) acc = gl::fp2_add(acc, gl::fp2_mul(ar[j], br[j]));
 #pragma unroll
         for (int m = 32; m > 0; m >>= 1) acc = gl::fp2_add(acc, fp2_shfl_xor(acc, m));
         if ((t & 63) == 0) part[t >> 6] = acc;
@@ -1057,9 +1132,21 @@ __global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __
             Fp2 s = part[0];
 #pragma unroll
             for (int w = 1; w < DOT_THREADS / 64; ++w) s = gl::fp2_add(s, part[w]);
-            out[row] = s;
+            out[row * gridDim.y + blockIdx.y] = s;
         }
         __syncthreads();
+    }
+}
+
+// out[row] = the sum of its `parts` partial dots, one wave per row.
+__global__ __launch_bounds__(64) void fp2_sum_parts_kernel(const Fp2* __restrict__ in, Fp2* __restrict__ out,
+                                                           size_t rows, size_t parts) {
+    for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        Fp2 acc{0, 0};
+        for (size_t i = threadIdx.x; i < parts; i += 64) acc = gl::fp2_add(acc, in[row * parts + i]);
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1) acc = gl::fp2_add(acc, fp2_shfl_xor(acc, m));
+        if (threadIdx.x == 0) out[row] = acc;
     }
 }
 
@@ -1067,11 +1154,13 @@ __global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __
 
 int eq_rows(Context* c, const Fp2* points, size_t rows, size_t dims, Fp2* out) {
     const int d = static_cast<int>(dims);
-    // Up to 16 outputs per thread, fewer when that would leave under 256
-    // threads (a single block claim's 2^9 weights: 256 threads of two,
-    // instead of 32 threads of sixteen running one serial wave).
+    // Up to 16 outputs per thread, fewer when that would leave under EQ_THREADS
+    // threads (one wave per SIMD): a thread is a serial chain of dims + 2^low
+    // products, and only a full machine hides it.  6 rows of 2^15: 17.2 -> 11.9
+    // us, one row of 2^11 12.4 -> 5.7.
+    constexpr size_t EQ_THREADS = 65536;
     int low = d < 4 ? d : 4;
-    while (low > 0 && (rows << (dims - low)) < 256) --low;
+    while (low > 0 && (rows << (dims - low)) < EQ_THREADS) --low;
     const size_t threads = rows << (dims - low);
     const dim3 grid(grid_for(threads, 256, 1 << 16));
     switch (low) {
@@ -1088,9 +1177,23 @@ int eq_rows(Context* c, const Fp2* points, size_t rows, size_t dims, Fp2* out) {
 int fp2_row_dots(Context* c, const Fp2* a, size_t a_stride, const Fp2* b, size_t b_stride, Fp2* out, size_t rows,
                  size_t len) {
     const unsigned blocks = static_cast<unsigned>(rows < 65535 ? rows : 65535);
-    hipLaunchKernelGGL(fp2_row_dots_kernel, dim3(blocks), dim3(DOT_THREADS), 0, c->stream, a, a_stride, b, b_stride,
-                       out, rows, len);
+    // Few long rows are cut into parts, about one workgroup per CU, whose sums a
+    // second launch adds.  6 rows of 2^15: 30.9 -> 10.7 us.  Inside a coarse timing
+    // scope, where workspaces may not grow, missing space leaves rows whole.
+    const size_t cus = c->cu_count > 0 ? static_cast<size_t>(c->cu_count) : 256;
+    size_t parts = rows < cus ? std::min(cus / rows, (len + DOT_PART - 1) / DOT_PART) : 1;
+    const size_t bytes = rows * parts * sizeof(Fp2);
+    if (parts > 1 && c->coarse_active && c->ws[WS_PARTIALS].capacity < bytes) parts = 1;
+    if (parts > 1 && ensure_ws(c, WS_PARTIALS, bytes)) return -1;
+    const size_t part_len = (len + parts - 1) / parts;
+    hipLaunchKernelGGL(fp2_row_dots_kernel, dim3(blocks, static_cast<unsigned>(parts)), dim3(DOT_THREADS), 0, c->stream,
+                       a, a_stride, b, b_stride, parts > 1 ? ws<Fp2>(c, WS_PARTIALS) : out, rows, len, part_len);
     VMX_HIP(c, hipGetLastError());
+    if (parts > 1) {
+        hipLaunchKernelGGL(fp2_sum_parts_kernel, dim3(blocks), dim3(64), 0, c->stream, ws<Fp2>(c, WS_PARTIALS), out,
+                           rows, parts);
+        VMX_HIP(c, hipGetLastError());
+    }
     return 0;
 }
 
