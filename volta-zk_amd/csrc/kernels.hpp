@@ -47,6 +47,13 @@ int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
 // The same for message rows lift(w) || pads || 0 of either size.
 int ntt_rr_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
                     uint64_t* out, TwiddleSet* t);
+// Rows of n = 2^8 .. 2^12 in one pass (ntt_small.hip): u64 rows as above, forward or
+// inverse (n^-1 scaled; len = n), and message rows.  1 (nothing done) for others and
+// for batches below 2^12 points a row that are too small to gain from it.
+int ntt_small_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, size_t n, uint64_t* out,
+                       TwiddleSet* t, bool inverse);
+int ntt_small_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
+                       uint64_t* out, TwiddleSet* t);
 // The n = 2^13 tables of ntt13r inside the encode's device table (built on
 // first use; null on error), and their builder.
 const uint64_t* enc13_rr_table(Context* c, TwiddleSet* t);

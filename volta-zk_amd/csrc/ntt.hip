@@ -176,6 +176,7 @@ int ntt_fp_rows(Context* c, const uint64_t* in, size_t in_stride, size_t msg_len
         if (rc <= 0) return rc;
     }
     if (t->reg) return reg_ntt(c, reg_tables(t), in, in_stride, msg_len, out, rows, ilog2(n), 1, inverse);
+    if (const int rc = ntt_small_u64_rows(c, in, in_stride, msg_len, rows, n, out, t, inverse); rc <= 0) return rc;
     const uint64_t scale = inverse ? gl::inv_host(gl::canon(n)) : 1;
     const uint64_t* tw = inverse ? t->inv : t->fwd;
     if (!tw) return fail_msg(c, "NTT twiddle table missing");
@@ -201,6 +202,7 @@ int ntt_msg_i16_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t 
         if (rc <= 0) return rc;
     }
     if (t->reg) return reg_ntt_msg_i16(c, reg_tables(t), w, pads, cols, pad, out, rows, ilog2(n));
+    if (const int rc = ntt_small_msg_rows(c, w, pads, cols, pad, rows, n, out, t); rc <= 0) return rc;
     return run_ntt(c, LoadMsgI16{w, pads, cols, pad}, StoreU64{out}, rows, n, t->fwd, 1);
 }
 
