@@ -288,6 +288,19 @@ def test_mobius_inverse_matches_oracle(backend, oracle, bits, off):
     assert np.array_equal(got[:off], guard[:off]) and np.array_equal(got[off + n:], guard[off + n:])
 
 
+@pytest.mark.parametrize("bits", [15, 16, 18, 19, 20, 21])
+def test_mobius_two_pass_splits(backend, oracle, bits):
+    """Both sides of each change of the two-pass split: eight bits in the second
+    pass from 2^16, longer runs at 2^20, nine bits at 2^21."""
+    from volta_mi355x import FP2
+    v = rand_fp2(bits + 300, 1 << bits)
+    d = backend.upload_device(v, FP2)
+    backend.fp2_mobius_inverse_inplace_device(d)
+    got = backend.download_device(d).view(np.uint64).reshape(-1, 2)
+    backend.free_device(d)
+    assert np.array_equal(got, oracle.fp2_mobius(v, inverse=True))
+
+
 # ---- geometry errors and stats ---------------------------------------------------------------
 
 def test_x4_geometry_errors(backend):

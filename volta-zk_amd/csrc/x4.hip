@@ -40,7 +40,10 @@ using u64x2 = uint64_t __attribute__((ext_vector_type(2)));
 using nreg::THREADS;
 constexpr int GBITS = nreg::GBITS;  // inner table: w_4096^j, j < 2048
 constexpr int TILE_BITS = 12;       // one-pass transforms and Moebius tiles: 2^12 Fp2 (64 KiB of LDS)
-constexpr int MOBIUS_RUN_BITS = 3;  // Moebius passes above the first: 8 adjacent columns
+constexpr int MOBIUS_RUN_BITS = 3;  // Moebius passes above the first: at least 8 adjacent columns
+// One group of a full tile's four-bit round per thread; two tiles fit a CU's LDS,
+// four waves per SIMD.  2^21 points: 256 threads 43.1 us, 512 33.7, 1024 43.6.
+constexpr int MOBIUS_THREADS = 512;
 constexpr uint64_t INV2 = 0x7FFFFFFF80000001ull;  // (p + 1) / 2
 using nreg::ROOT33_C1;
 using nreg::Digits;
@@ -107,25 +110,34 @@ __global__ __launch_bounds__(THREADS) void direct_fold(const u64x2* __restrict__
     uint64_t j = static_cast<uint64_t>(blockIdx.x) * THREADS + threadIdx.x;
     if (j >= count) return;
     const uint64_t mask = (uint64_t{1} << nb) - 1;
+    u64x2 p = pos[j], q = neg[j];  // in flight while the twiddle is formed
     bool imag;
     uint64_t y = halve(root_pow((uint64_t{0} - (j0 + j)) & mask, nb, split, h, imag));
-    for (; j < count; j += D) {
-        const u64x2 p = pos[j], q = neg[j];
+    for (;;) {
         const u64x2 even{halve(gl::add(p.x, q.x)), halve(gl::add(p.y, q.y))};
         const u64x2 dd{gl::sub(p.x, q.x), gl::sub(p.y, q.y)};
         const u64x2 odd = imag ? u64x2{mul7(gl::mul32x4(dd.y, y)), gl::mul32x4(dd.x, y)}
                                : u64x2{gl::mul32x4(dd.x, y), gl::mul32x4(dd.y, y)};
         const u64x2 co = fp2_mul(ch, odd);
         out[j] = u64x2{gl::add(even.x, co.x), gl::add(even.y, co.y)};
+        j += D;
+        if (j >= count) return;
+        p = pos[j];
+        q = neg[j];
         y = gl::mul32x4(y, step);
     }
 }
 
 // ---- Moebius transform -------------------------------------------------------------------
 
-// LDS word of tile index i: one word of padding per 16 keeps the rounds below
-// free of bank conflicts (a round's lanes step by 1, 17 or 272 words).
-__device__ __forceinline__ uint32_t mob_slot(uint32_t i) { return i + (i >> 4); }
+// LDS word of element i of plane-column pc: one word of padding per 16 keeps
+// the rounds below free of bank conflicts (a round's lanes step by 1, 17 or 272
+// words), four more per plane-column those of the loads and stores (eight
+// adjacent columns of four elements in 32 lanes).
+__device__ __forceinline__ uint32_t mob_slot(uint32_t pc, uint32_t i, int rb) {
+    const uint32_t e = (pc << rb) + i;
+    return e + (e >> 4) + 4 * pc;
+}
 
 // One round of the Moebius transform on the tile in LDS: bits [b, b + K) of
 // the middle index, all K of them in registers.  Group g takes the 2^K
@@ -135,13 +147,13 @@ template <int K>
 __device__ __forceinline__ void mobius_round(uint64_t* s, int b, int rb, uint32_t planecols, int inverse) {
     const uint32_t lo_mask = (1u << b) - 1, hi_bits = static_cast<uint32_t>(rb - b - K);
     const uint32_t groups = planecols << (rb - K);
-    for (uint32_t g = threadIdx.x; g < groups; g += THREADS) {
+    for (uint32_t g = threadIdx.x; g < groups; g += MOBIUS_THREADS) {
         const uint32_t lo = g & lo_mask, hi = (g >> b) & ((1u << hi_bits) - 1), pc = g >> (rb - K);
-        const uint32_t i0 = (pc << rb) + lo + (hi << (b + K));
+        const uint32_t i0 = lo + (hi << (b + K));
         uint64_t v[1 << K];
         gl::static_for<0, (1 << K)>([&](auto m_) {
             constexpr int m = decltype(m_)::value;
-            v[m] = s[mob_slot(i0 + (static_cast<uint32_t>(m) << b))];
+            v[m] = s[mob_slot(pc, i0 + (static_cast<uint32_t>(m) << b), rb)];
         });
         gl::static_for<0, K>([&](auto j_) {
             constexpr int j = decltype(j_)::value;
@@ -152,7 +164,7 @@ __device__ __forceinline__ void mobius_round(uint64_t* s, int b, int rb, uint32_
         });
         gl::static_for<0, (1 << K)>([&](auto m_) {
             constexpr int m = decltype(m_)::value;
-            s[mob_slot(i0 + (static_cast<uint32_t>(m) << b))] = v[m];
+            s[mob_slot(pc, i0 + (static_cast<uint32_t>(m) << b), rb)] = v[m];
         });
     }
 }
@@ -161,7 +173,7 @@ __device__ __forceinline__ void mobius_round(uint64_t* s, int b, int rb, uint32_
 // bit of i, the element with the bit set gains (inverse) or loses the one
 // without.  Workgroup (h, l0) takes C = 2^cb adjacent columns; the bits are
 // applied up to four at a time in registers, with the tile in LDS in between.
-__global__ __launch_bounds__(THREADS) void mobius_pass(u64x2* a, int rb, int lb, int cb, int inverse) {
+__global__ __launch_bounds__(MOBIUS_THREADS) void mobius_pass(u64x2* a, int rb, int lb, int cb, int inverse) {
     extern __shared__ uint64_t s[];
     const uint32_t C = 1u << cb;
     const uint32_t CR = C << rb;
@@ -169,11 +181,11 @@ __global__ __launch_bounds__(THREADS) void mobius_pass(u64x2* a, int rb, int lb,
     const uint64_t h = blockIdx.x / lblocks;
     const uint64_t l0 = (blockIdx.x - h * lblocks) << cb;
     const uint64_t base = ((h << rb) << lb) + l0;
-    for (uint32_t e = threadIdx.x; e < CR; e += THREADS) {
+    for (uint32_t e = threadIdx.x; e < CR; e += MOBIUS_THREADS) {
         const uint32_t i = e >> cb, c = e & (C - 1);
         const u64x2 v = a[base + (static_cast<uint64_t>(i) << lb) + c];
-        s[mob_slot((c << rb) + i)] = v.x;
-        s[mob_slot(CR + (c << rb) + i)] = v.y;
+        s[mob_slot(c, i, rb)] = v.x;
+        s[mob_slot(C + c, i, rb)] = v.y;
     }
     __syncthreads();
     for (int b = 0; b < rb; b += 4) {
@@ -185,9 +197,9 @@ __global__ __launch_bounds__(THREADS) void mobius_pass(u64x2* a, int rb, int lb,
         }
         __syncthreads();
     }
-    for (uint32_t e = threadIdx.x; e < CR; e += THREADS) {
+    for (uint32_t e = threadIdx.x; e < CR; e += MOBIUS_THREADS) {
         const uint32_t i = e >> cb, c = e & (C - 1);
-        a[base + (static_cast<uint64_t>(i) << lb) + c] = u64x2{s[mob_slot((c << rb) + i)], s[mob_slot(CR + (c << rb) + i)]};
+        a[base + (static_cast<uint64_t>(i) << lb) + c] = u64x2{s[mob_slot(c, i, rb)], s[mob_slot(C + c, i, rb)]};
     }
 }
 
@@ -298,22 +310,33 @@ int fp2_mobius(Context* c, gl::Fp2* values, uint64_t n, bool inverse) {
     using namespace x4;
     const int nb = log2_exact(n);
     auto* a = reinterpret_cast<u64x2*>(values);
-    // low bits first: contiguous tiles of up to 2^12; then the bits above in
-    // passes of up to 2^10 over 4 adjacent columns
-    int done = 0;
+    // Low bits first: contiguous tiles, then the bits above in even passes over
+    // runs of adjacent columns.  Up to 2^12 points take one tile.  Up to 2^20 two
+    // passes of about half the bits (at most eight above: two rounds), so that
+    // small transforms have many workgroups; from 2^21 on full tiles, where a pass
+    // of few bits takes longer runs.  Against 12 bits first, the rest nine at a
+    // time over runs of eight, 256 threads, us: 2^12 14.1 -> 9.2, 2^13 18.9 -> 8.6,
+    // 2^16 21.0 -> 12.9, 2^18 24.0 -> 16.1, 2^20 32.6 -> 27.1, 2^21 43.1 -> 33.7,
+    // 2^22 203 -> 82 and 2^23 290 -> 157 (three passes: 4.9 and 5.1 TB/s).
+    const int first = nb <= TILE_BITS ? nb : std::max(nb - 8, (nb + 1) / 2);
+    const int r0 = std::min(first, TILE_BITS);
+    const int above = (nb - r0 + TILE_BITS - MOBIUS_RUN_BITS - 1) / (TILE_BITS - MOBIUS_RUN_BITS);
+    int done = 0, pass = 0;
     while (done < nb) {
         const int lb = done;
-        const int cb = std::min(MOBIUS_RUN_BITS, lb);
-        const int rb = std::min(nb - done, TILE_BITS - cb);
+        const int rb = pass == 0 ? r0 : (nb - r0) / above + (pass <= (nb - r0) % above ? 1 : 0);
+        // runs of eight columns at least, longer while 256 workgroups remain
+        const int cb = std::min(lb, std::max(MOBIUS_RUN_BITS, std::min(TILE_BITS - rb, nb - rb - 8)));
         const uint64_t blocks = uint64_t{1} << (nb - rb - cb);
         const size_t words = size_t{2} << (rb + cb);  // two planes
-        const size_t lds = (words + (words >> 4) + 1) * sizeof(uint64_t);  // + the slots' padding
+        const size_t lds = (words + (words >> 4) + 1 + (size_t{8} << cb)) * sizeof(uint64_t);  // + the slots' padding
         if (blocks > 0x7FFFFFFFull) return fail_msg(c, "Moebius pass exceeds its launch limits");
         if (set_lds(c, mobius_pass, lds)) return -1;
-        hipLaunchKernelGGL(mobius_pass, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), lds, c->stream, a, rb,
+        hipLaunchKernelGGL(mobius_pass, dim3(static_cast<unsigned>(blocks)), dim3(MOBIUS_THREADS), lds, c->stream, a, rb,
                            lb, cb, inverse ? 1 : 0);
         VMX_HIP(c, hipGetLastError());
         done += rb;
+        ++pass;
     }
     return 0;
 }
