@@ -36,3 +36,33 @@ def test_chunk_runs(backend, oracle, rows, bits):
     got = tree_of(backend, m)
     leaves = oracle.hash_fp_columns(m, rows, 1 << bits)
     assert (got[:1 << bits] == leaves.reshape(-1, 32)).all()
+
+
+def hash_in_scope(b, rows, cols, seed):
+    """(tree, matrix) of a hash inside a coarse timing scope, where nothing may be allocated."""
+    m = np.random.Generator(np.random.PCG64(seed)).integers(0, P, size=(rows, cols), dtype=np.uint64)
+    buf, tree = b.upload_device(m.reshape(-1)), b.alloc_device((2 * cols - 1) * 32, np.uint8)
+    live = b.get_stats()["live_device_bytes"]
+    assert b.lib.volta_cuda_begin_coarse_timing(b.raw, 4) == 0
+    rc = b.lib.volta_cuda_hash_fp_tree_device(b.raw, buf.id, 0, rows, cols, tree.id, 0)
+    assert rc == 0, b.last_error()
+    assert b.lib.volta_cuda_end_coarse_timing(b.raw) == 0
+    assert b.get_stats()["live_device_bytes"] == live
+    got = b.download_device(tree).reshape(-1, 32)
+    for x in (buf, tree):
+        b.free_device(x)
+    return got, m
+
+
+# columns of up to four chunks need no workspace as one run, so a new context
+# hashes them inside a scope; after columns of five chunks (two runs of at most
+# four) there is space for columns of eight
+@pytest.mark.parametrize("warm,rows", [(0, 129), (0, 300), (0, 512), (520, 1024)])
+def test_hash_where_workspaces_may_not_grow(oracle, warm, rows):
+    from volta_mi355x import Backend
+    cols = 1 << 10
+    with Backend(timing_policy=1) as b:
+        if warm:
+            tree_of(b, np.ones((warm, cols), np.uint64))
+        got, m = hash_in_scope(b, rows, cols, rows)
+    assert (got == oracle.merkle_tree(oracle.hash_fp_columns(m, rows, cols)).reshape(-1, 32)).all()

@@ -312,6 +312,32 @@ int ensure_ws(Context* c, int slot, size_t bytes) {
     return 0;
 }
 
+bool try_ws(Context* c, int slot, size_t bytes) {
+    Workspace& w = c->ws[slot];
+    if (w.capacity >= bytes) return true;
+    if (c->coarse_active) return false;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {  // the old space is still there for the slower way
+        (void)hipGetLastError();
+        return false;
+    }
+    ++c->stats.allocation_calls;
+    c->stats.live_device_bytes += bytes;
+    c->stats.peak_device_bytes = std::max(c->stats.peak_device_bytes, c->stats.live_device_bytes);
+    if (w.ptr) {
+        if (sync_stream(c, SyncReason::AllocatorFlush) || hipFree(w.ptr) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(p);
+            c->stats.live_device_bytes -= bytes;
+            return false;
+        }
+        ++c->stats.physical_free_calls;
+        c->stats.live_device_bytes -= w.capacity;
+    }
+    w = Workspace{p, bytes};
+    return true;
+}
+
 static int upload_table(Context* c, const std::vector<uint64_t>& host, uint64_t** out,
                         uint64_t* h2d) {
     const size_t bytes = host.size() * sizeof(uint64_t);

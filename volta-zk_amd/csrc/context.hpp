@@ -351,6 +351,9 @@ int staged_copy(Context* c, void* dst, const void* src, size_t bytes, hipMemcpyK
 
 // ---- workspaces and twiddles ---------------------------------------------------
 int ensure_ws(Context* c, int slot, size_t bytes);
+// The same for space that only a faster way needs: false, with nothing changed,
+// where it may not grow (inside a coarse timing scope) or memory is short.
+bool try_ws(Context* c, int slot, size_t bytes);
 template <typename T>
 T* ws(Context* c, int slot) {
     return static_cast<T*>(c->ws[slot].ptr);

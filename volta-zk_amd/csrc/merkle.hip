@@ -562,19 +562,25 @@ int merkle_column_leaves(Context* c, const uint64_t* m, size_t rows, size_t cols
     const size_t w = fp2 ? 2 : 1;
     const size_t words = rows * w;
     const size_t chunks = (words + b3::CHUNK_WORDS - 1) / b3::CHUNK_WORDS;
-    const size_t group = chunks_per_thread(c, cols, chunks);
-    size_t k = (chunks + group - 1) / group;           // values per column after column_groups
-    if (k > 65535) return fail_msg(c, "Merkle column too long (more than 2^18 BLAKE3 chunks)");
-    // workspace: column_groups' values, then each non-final merge pass's (16x fewer)
-    size_t slots = 0;
-    for (size_t kk = k; kk > 1; kk = (kk + b3::FAN_IN - 1) / b3::FAN_IN) slots += kk;
-    uint32_t* buf = nullptr;
-    if (k > 1) {
-        size_t bytes = 0;
-        if (!mul_ok(slots, cols * 32, &bytes)) return fail_msg(c, "Merkle workspace overflows size_t");
-        if (ensure_ws(c, WS_HASH, bytes)) return -1;
-        buf = ws<uint32_t>(c, WS_HASH);
+    if (chunks > 4 * size_t{65535}) return fail_msg(c, "Merkle column too long (more than 2^18 BLAKE3 chunks)");
+    // Workspace of runs of `g` chunks: column_groups' values, then each non-final merge
+    // pass's (16x fewer).
+    auto ws_bytes = [&](size_t g, size_t* bytes) {
+        size_t slots = 0;
+        for (size_t kk = (chunks + g - 1) / g; kk > 1; kk = (kk + b3::FAN_IN - 1) / b3::FAN_IN) slots += kk;
+        return mul_ok(slots, cols * 32, bytes);
+    };
+    size_t group = chunks_per_thread(c, cols, chunks), bytes = 0;
+    // Short runs leave more values: where the workspace for them is not to be had, as
+    // inside a coarse timing scope, the longest runs do, which need the least (none up
+    // to four chunks).
+    if (!ws_bytes(group, &bytes) || !try_ws(c, WS_HASH, bytes)) {
+        group = std::min<size_t>(4, chunks);
+        if (!ws_bytes(group, &bytes)) return fail_msg(c, "Merkle workspace overflows size_t");
     }
+    size_t k = (chunks + group - 1) / group;  // values per column after column_groups
+    if (bytes && ensure_ws(c, WS_HASH, bytes)) return -1;
+    uint32_t* buf = bytes ? ws<uint32_t>(c, WS_HASH) : nullptr;
     const dim3 grid(static_cast<unsigned>((cols + b3::LANES - 1) / b3::LANES), static_cast<unsigned>(k));
     const int is_root = k == 1 ? 1 : 0;
     uint32_t* gout = k == 1 ? leaves : buf;
