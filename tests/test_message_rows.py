@@ -44,11 +44,14 @@ def test_emulated_rows(bits, cols, pad):
     assert (got == want.reshape(rows, n)).all()
 
 
+# row counts on both sides of where the one pass takes over from the pass engine's two
+# (5/8 of 256 CUs at 2^13, half of them at 2^14), and more rows than workgroups
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits,cols,pad", SHAPES)
-@pytest.mark.parametrize("rows", [1, 1030])
+@pytest.mark.parametrize("rows", [1, -1, 0, 1030])
 def test_device_rows(backend, bits, cols, pad, rows):
     n = 1 << bits
+    rows = rows if rows > 0 else (160 if bits == 13 else 128) + rows
     w, pads = inputs(rows, cols, pad)
     dw, dp = backend.upload_device(w.reshape(-1)), backend.upload_device(pads.reshape(-1))
     msgs = backend.pcs_messages_device(dw, 0, dp, 0, rows, cols, pad, n)

@@ -212,12 +212,23 @@ int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
     return rr::u64_rows<4>(c, in, stride, len, rows, t->grid, out);
 }
 
+// A row is one workgroup's chain of three stages, which the pass engine spreads over
+// 16 to 32 workgroups a pass: message rows take this way once they fill 5/8 (2^13)
+// or half (2^14) of the CUs.  Pass engine and one pass, us: 2^13, 2,048 + 512: 64 rows
+// 13.5 / 17.8, 128 17.2 / 17.9, 160 19.3 / 17.9; 1,000 + 77: 144 18.6 / 19.0, 160
+// 19.0 / 18.9; 2^14, 4,096 + 512: 64 rows 19.2 / 22.5, 96 22.3 / 22.6, 112 24.8 / 23.1;
+// 1,000 + 77: 112 23.9 / 24.6, 128 25.1 / 25.1; one row of either 11.7 / 17.0 and
+// 13.3 / 21.5.
+static bool msg_pays(const Context* c, size_t rows, bool b3) {
+    const size_t cus = c->cu_count > 0 ? static_cast<size_t>(c->cu_count) : 256;
+    return b3 ? rows >= cus * 5 / 8 : rows >= cus / 2;
+}
+
 int ntt_rr_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
                     uint64_t* out, TwiddleSet* t) {
     const bool b3 = n == static_cast<size_t>(rr::Shape<3>::N), b4 = n == static_cast<size_t>(rr::Shape<4>::N);
-    if ((!b3 && !b4) || cols == 0 || cols + pad > n || !t->fwd) return 1;
+    if ((!b3 && !b4) || !msg_pays(c, rows, b3) || cols == 0 || cols + pad > n || !t->fwd) return 1;
     if (!t->grid && c->coarse_active) return 1;
-    if (rows == 0) return 0;
     if (b3) {
         const uint64_t* tab = enc13_rr_table(c, t);
         if (!tab) return -1;
