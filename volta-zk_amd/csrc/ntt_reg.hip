@@ -138,6 +138,17 @@ constexpr int parked() {  // outputs per step-1 job in LDS at a time
     return two_rounds<LA>() ? 16 : 1 << LA;
 }
 
+// threadIdx.x as the compiler cannot know it from before: what is computed from it
+// is computed after this point instead of being held in registers across it.  The
+// two-round kernels otherwise keep step 2's addresses through step 1 and spill (13
+// words in the u64 gather, 4 in the column pass without a table): 2^18 x 16 rows,
+// gather 30 -> 24.3 us with no scratch.
+__device__ __forceinline__ uint32_t here() {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 // Step 2's head: the B values of (pc, ka), DFT'd over jb (natural order over kb);
 // the outputs in NEED are canonical.
 template <int LB, uint64_t NEED>
@@ -177,6 +188,8 @@ struct SrcU64 {
     __device__ __forceinline__ uint32_t rotation() const { return reverse ? 1u : 0u; }
     // A tile's u64 runs are whole lines: tiles go to the XCDs round-robin.
     static constexpr bool SWIZZLE = false;
+    // Inputs of a two-round job whose loads are in flight together.
+    static constexpr int IN_FLIGHT = 32;
     __device__ __forceinline__ Raw fetch(uint64_t row, uint64_t idx, uint32_t plane, int PL) const {
         const uint64_t ci = idx < len ? idx : 0;
         return Raw{x[(row * x_stride + ci) * PL + plane]};
@@ -206,6 +219,8 @@ struct SrcMsgI16 {
     // A tile's i16 runs are 32 bytes, a quarter of a line: consecutive tiles
     // run on one XCD so that the line is fetched into its L2 once.
     static constexpr bool SWIZZLE = true;
+    // Two words per input: all 32 at once took 27 words of scratch.
+    static constexpr int IN_FLIGHT = 16;
     __device__ __forceinline__ Raw fetch(uint64_t row, uint64_t idx, uint32_t, int) const {
         const uint64_t wi = idx < cols ? idx : 0;
         const uint64_t pi = idx >= cols && idx - cols < pad ? idx - cols : 0;
@@ -280,17 +295,21 @@ __global__ __launch_bounds__(THREADS, two_rounds<LA>() ? 4 : 1) void gather_reg(
     auto step1 = [&](uint32_t pc, uint32_t jb, uint64_t* v) {
         const uint32_t plane = PL == 2 ? (pc & 1) : 0, t = PL == 2 ? (pc >> 1) : pc;
         const uint64_t L = (nat0 + t + rot) & lmask;
-        typename Src::Raw raw[NZ];
-        gl::static_for<0, NZ>([&](auto ja_) {
-            constexpr int ja = decltype(ja_)::value;
-            const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
-            raw[ja] = src.fetch(row, idx, plane, PL);
-        });
         gl::static_for<0, A>([&](auto i_) { v[decltype(i_)::value] = 0; });
-        gl::static_for<0, NZ>([&](auto ja_) {
-            constexpr int ja = decltype(ja_)::value;
-            const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
-            v[gl::bitrev_c(ja, LA)] = src.finish(idx, raw[ja]);
+        constexpr int BATCH = two_rounds<LA>() ? std::min(NZ, Src::IN_FLIGHT) : NZ;
+        gl::static_for<0, (NZ + BATCH - 1) / BATCH>([&](auto q_) {
+            constexpr int j0 = BATCH * decltype(q_)::value, j1 = std::min(j0 + BATCH, NZ);
+            typename Src::Raw raw[j1 - j0];
+            gl::static_for<j0, j1>([&](auto ja_) {
+                constexpr int ja = decltype(ja_)::value;
+                const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
+                raw[ja - j0] = src.fetch(row, idx, plane, PL);
+            });
+            gl::static_for<j0, j1>([&](auto ja_) {
+                constexpr int ja = decltype(ja_)::value;
+                const uint64_t idx = src.index(L + ((static_cast<uint64_t>(ja) * B + jb) << sh), nmask);
+                v[gl::bitrev_c(ja, LA)] = src.finish(idx, raw[ja - j0]);
+            });
         });
         gl::dit_pow2_sparse<LA, ew_log<LA>(), prefix_mask(NZ, LA), 2, (2 << LA), 1>(v);  // park() twiddles all but v[0]
     };
@@ -313,12 +332,12 @@ __global__ __launch_bounds__(THREADS, two_rounds<LA>() ? 4 : 1) void gather_reg(
         step1(job & 15, job >> 4, v);
         park<LA, LB, 0, 16>(s, v, job & 15, job >> 4, PW, pitch, ptw);
         __syncthreads();
-        step2(job >> 4, job & 15, 0);
+        step2(here() >> 4, here() & 15, 0);
         __syncthreads();
-        park<LA, LB, 16, 16>(s, v, job & 15, job >> 4, PW, pitch, ptw);
+        park<LA, LB, 16, 16>(s, v, here() & 15, here() >> 4, PW, pitch, ptw);
         __syncthreads();
         __builtin_amdgcn_s_setprio(0);
-        step2(job >> 4, 16 + (job & 15), 16);
+        step2(here() >> 4, 16 + (here() & 15), 16);
     } else {
         for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
             const uint32_t pc = job & (PW - 1), jb = job >> pwb;
@@ -506,16 +525,17 @@ __global__ __launch_bounds__(THREADS, two_rounds<LA>() ? 4 : 1) void col_reg(uin
     };
     if constexpr (two_rounds<LA>()) {
         const uint32_t pc = threadIdx.x & 15, q = threadIdx.x >> 4;
+        auto at = [] { return TBL ? threadIdx.x : here(); };
         uint64_t v[A];
         step1(pc, q, v);
         park<LA, LB, 0, 16>(s, v, pc, q, PW, pitch, ptw);
         __syncthreads();
-        step2(pc, q, 0);
+        step2(at() & 15, at() >> 4, 0);
         __syncthreads();
-        park<LA, LB, 16, 16>(s, v, pc, q, PW, pitch, ptw);
+        park<LA, LB, 16, 16>(s, v, at() & 15, at() >> 4, PW, pitch, ptw);
         __syncthreads();
         __builtin_amdgcn_s_setprio(0);
-        step2(pc, 16 + q, 16);
+        step2(at() & 15, 16 + (at() >> 4), 16);
     } else {
         for (uint32_t job = threadIdx.x; job < (PW << LB); job += THREADS) {
             const uint32_t pc = job & (PW - 1), jb = job >> pwb;
