@@ -17,7 +17,8 @@ def fp2(seed, n):
     return np.random.default_rng(seed).integers(0, P, size=(n, 2), dtype=np.uint64)
 
 
-@pytest.mark.parametrize("rows,count", [(1, 8192), (2, 8193), (7, 66561), (1024, 8199), (1025, 8192), (3, 511), (5, 1024)])
+@pytest.mark.parametrize("rows,count", [(1, 8192), (2, 8193), (7, 66561), (1024, 8199), (1025, 8192), (3, 511), (5, 1024),
+                                        (2, 1537), (7, 4097)])
 def test_long_rows_with_and_without_a_rejection(backend, oracle, rows, count):
     for domain in (0x19664BCA, 0x19664BCB, 0x19664BCA):  # a rejected row, none, and again
         d = backend.chacha8_prover_secret_fp_rows_device(KAT_SEED, domain, rows, count)
