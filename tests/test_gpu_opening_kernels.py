@@ -27,7 +27,7 @@ def test_long_rows_with_and_without_a_rejection(backend, oracle, rows, count):
         assert (got == oracle.fp_rows(KAT_SEED, domain, rows, count)).all()
 
 
-@pytest.mark.parametrize("rows,dims", [(1, 0), (1, 1), (1, 16), (6, 15), (1, 17), (3, 17), (64, 13), (97, 13)])
+@pytest.mark.parametrize("rows,dims", [(1, 0), (1, 1), (1, 16), (6, 15), (1, 17), (3, 17), (64, 13), (97, 13), (129, 13)])
 def test_equality_rows(backend, oracle, rows, dims):
     pts = fp2(rows + dims, rows * dims)
     buf = backend.upload_device(pts, pts_dtype()) if dims else None

@@ -1072,8 +1072,12 @@ __global__ __launch_bounds__(256) void eq_rows_kernel(const Fp2* __restrict__ po
         const Fp2* p = points + r * dims;
         Fp2 v[1 << LOW];
         v[0] = Fp2{1, 0};
+        // each factor is loaded one product ahead: 3 rows of 2^19 25.0 -> 21.8 us, 2^21 27.4
+        // -> 24.8 (two waves per SIMD, which do not hide the loads)
+        Fp2 next = LOW < dims ? p[LOW] : v[0];
         for (int k = LOW; k < dims; ++k) {
-            const Fp2 pk = p[k];
+            const Fp2 pk = next;
+            if (k + 1 < dims) next = p[k + 1];
             v[0] = gl::fp2_mul(v[0], ((hi >> (k - LOW)) & 1) ? pk : fp2_one_minus(pk));
         }
 #pragma unroll
