@@ -1,7 +1,8 @@
 """The opening's small kernels at the edges of their dispatch, bit-exact against
 the oracle: mask rows spread over the GPU and their rejected draws, equality
-rows with each number of outputs per thread, dots of whole and of cut rows; and
-the first two inside a coarse timing scope, where workspaces may not grow."""
+rows with each number of outputs per thread, dots of whole, of cut and of many
+short rows; mask rows and dots also inside a coarse timing scope, where
+workspaces may not grow."""
 import numpy as np
 import pytest
 
@@ -46,7 +47,8 @@ def pts_dtype():
 
 
 @pytest.mark.parametrize("rows,length", [(1, 1), (1, 4096), (1, 4097), (1, 100000), (6, 32768), (97, 8200), (255, 8193),
-                                         (256, 8193), (300, 5000)])
+                                         (256, 8193), (300, 5000), (1, 8191), (1, 8192), (128, 8192), (256, 512),
+                                         (257, 1), (257, 512), (257, 513), (3000, 300)])
 def test_row_dots(backend, oracle, rows, length):
     stride = length + 3
     a, b = fp2(length, rows * stride), fp2(length + 1, rows * length)

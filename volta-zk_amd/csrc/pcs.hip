@@ -1099,6 +1099,8 @@ __global__ __launch_bounds__(256) void eq_rows_kernel(const Fp2* __restrict__ po
 }
 
 constexpr int DOT_THREADS = 1024;  // 16 waves per row: a claim's mask row is 2^13..2^17 long
+constexpr int DOT_SHORT_THREADS = 256;  // many rows of up to DOT_SHORT elements
+constexpr size_t DOT_SHORT = 512;
 constexpr int DOT_UNROLL = 4;      // products whose loads are in flight together
 constexpr size_t DOT_PART = size_t{DOT_THREADS} * DOT_UNROLL;  // least elements of a part
 
@@ -1109,30 +1111,32 @@ __device__ __forceinline__ Fp2 fp2_shfl_xor(Fp2 x, int m) {
 
 // out[r] = sum_j a[r a_stride + j] b[r b_stride + j] (reference .cu:1374-1391):
 // one workgroup per row, strided partial sums, a shuffle reduction inside each
-// wave and one LDS step across the four waves.
-__global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __restrict__ a, size_t a_stride,
-                                                                   const Fp2* __restrict__ b, size_t b_stride,
-                                                                   Fp2* __restrict__ out, size_t rows, size_t len,
-                                                                   size_t part_len) {
-    __shared__ Fp2 part[DOT_THREADS / 64];
+// wave and one LDS step across the waves.  With CUT, workgroup (r, part) takes
+// part_len of the row's products and writes out[r parts + part].
+template <int THREADS, bool CUT>
+__global__ __launch_bounds__(THREADS) void fp2_row_dots_kernel(const Fp2* __restrict__ a, size_t a_stride,
+                                                               const Fp2* __restrict__ b, size_t b_stride,
+                                                               Fp2* __restrict__ out, size_t rows, size_t len,
+                                                               size_t part_len) {
+    __shared__ Fp2 part[THREADS / 64];
     const int t = threadIdx.x;
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         Fp2 acc{0, 0};
         const Fp2* ar = a + row * a_stride;
         const Fp2* br = b + row * b_stride;
-        size_t j = blockIdx.y * part_len + t;
-        const size_t end = min(len, (blockIdx.y + 1) * part_len);
-        for (; j + (DOT_UNROLL - 1) * DOT_THREADS < end; j += DOT_UNROLL * DOT_THREADS) {
+        size_t j = CUT ? blockIdx.y * part_len + t : t;
+        const size_t end = CUT ? min(len, (blockIdx.y + 1) * part_len) : len;
+        for (; j + (DOT_UNROLL - 1) * THREADS < end; j += DOT_UNROLL * THREADS) {
             Fp2 x[DOT_UNROLL], y[DOT_UNROLL];
 #pragma unroll
             for (int u = 0; u < DOT_UNROLL; ++u) {
-                x[u] = ar[j + u * DOT_THREADS];
-                y[u] = br[j + u * DOT_THREADS];
+                x[u] = ar[j + u * THREADS];
+                y[u] = br[j + u * THREADS];
             }
 #pragma unroll
             for (int u = 0; u < DOT_UNROLL; ++u) acc = gl::fp2_add(acc, gl::fp2_mul(x[u], y[u]));
         }
-        for (; j < end; j += DOT_THREADS) acc = gl::fp2_add(acc, gl::fp2_mul(ar[j], br[j]));
+        for (; j < end; j += THREADS) acc = gl::fp2_add(acc, gl::fp2_mul(ar[j], br[j]));
 #pragma unroll
         for (int m = 32; m > 0; m >>= 1) acc = gl::fp2_add(acc, fp2_shfl_xor(acc, m));
         if ((t & 63) == 0) part[t >> 6] = acc;
@@ -1140,8 +1144,8 @@ __global__ __launch_bounds__(DOT_THREADS) void fp2_row_dots_kernel(const Fp2* __
         if (t == 0) {
             Fp2 s = part[0];
 #pragma unroll
-            for (int w = 1; w < DOT_THREADS / 64; ++w) s = gl::fp2_add(s, part[w]);
-            out[row * gridDim.y + blockIdx.y] = s;
+            for (int w = 1; w < THREADS / 64; ++w) s = gl::fp2_add(s, part[w]);
+            out[CUT ? row * gridDim.y + blockIdx.y : row] = s;
         }
         __syncthreads();
     }
@@ -1187,22 +1191,32 @@ int fp2_row_dots(Context* c, const Fp2* a, size_t a_stride, const Fp2* b, size_t
                  size_t len) {
     const unsigned blocks = static_cast<unsigned>(rows < 65535 ? rows : 65535);
     // Few long rows are cut into parts, about one workgroup per CU, whose sums a
-    // second launch adds.  6 rows of 2^15: 30.9 -> 10.7 us.  Inside a coarse timing
-    // scope, where workspaces may not grow, missing space leaves rows whole.
+    // second launch adds.  6 rows of 2^15: 30.9 -> 10.7 us; of 8,192 10.1 -> 9.8, but of
+    // 4,097 7.1 -> 8.5 and of 6,000 8.6 -> 9.1, which the second launch costs.  Without
+    // the space for the parts (it may not grow inside a coarse timing scope) rows stay
+    // whole.
     const size_t cus = c->cu_count > 0 ? static_cast<size_t>(c->cu_count) : 256;
-    size_t parts = rows < cus ? std::min(cus / rows, (len + DOT_PART - 1) / DOT_PART) : 1;
-    const size_t bytes = rows * parts * sizeof(Fp2);
-    if (parts > 1 && c->coarse_active && c->ws[WS_PARTIALS].capacity < bytes) parts = 1;
-    if (parts > 1 && ensure_ws(c, WS_PARTIALS, bytes)) return -1;
-    const size_t part_len = (len + parts - 1) / parts;
-    hipLaunchKernelGGL(fp2_row_dots_kernel, dim3(blocks, static_cast<unsigned>(parts)), dim3(DOT_THREADS), 0, c->stream,
-                       a, a_stride, b, b_stride, parts > 1 ? ws<Fp2>(c, WS_PARTIALS) : out, rows, len, part_len);
-    VMX_HIP(c, hipGetLastError());
-    if (parts > 1) {
+    const size_t parts =
+        rows < cus && len >= 2 * DOT_PART ? std::min(cus / rows, (len + DOT_PART - 1) / DOT_PART) : 1;
+    if (parts > 1 && try_ws(c, WS_PARTIALS, rows * parts * sizeof(Fp2))) {
+        hipLaunchKernelGGL((fp2_row_dots_kernel<DOT_THREADS, true>), dim3(blocks, static_cast<unsigned>(parts)), dim3(DOT_THREADS), 0,
+                           c->stream, a, a_stride, b, b_stride, ws<Fp2>(c, WS_PARTIALS), rows, len,
+                           (len + parts - 1) / parts);
+        VMX_HIP(c, hipGetLastError());
         hipLaunchKernelGGL(fp2_sum_parts_kernel, dim3(blocks), dim3(64), 0, c->stream, ws<Fp2>(c, WS_PARTIALS), out,
                            rows, parts);
-        VMX_HIP(c, hipGetLastError());
+    } else {
+        auto whole = [&](auto kernel, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, c->stream, a, a_stride, b, b_stride, out, rows,
+                               len, len);
+        };
+        // More short rows than CUs: the 16-wave workgroups would mostly reduce zeros.
+        // 1,000 rows of 100 7.2 -> 4.6 us, of 512 7.7 -> 5.1; 300 of 1 4.8 -> 4.6, but of
+        // 897 5.7 / 5.7, where a workgroup takes both loops.
+        if (rows > cus && len <= DOT_SHORT) whole(fp2_row_dots_kernel<DOT_SHORT_THREADS, false>, DOT_SHORT_THREADS);
+        else whole(fp2_row_dots_kernel<DOT_THREADS, false>, DOT_THREADS);
     }
+    VMX_HIP(c, hipGetLastError());
     return 0;
 }
 
