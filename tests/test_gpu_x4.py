@@ -270,7 +270,7 @@ def test_x4_fold_pinned_tile_errors(backend):
 
 # ---- Moebius inverse --------------------------------------------------------------------------
 
-@pytest.mark.parametrize("bits,off", [(0, 0), (1, 0), (2, 1), (5, 0), (11, 3), (12, 0), (13, 0), (14, 2), (17, 0),
+@pytest.mark.parametrize("bits,off", [(0, 0), (1, 0), (2, 1), (5, 0), (8, 0), (9, 2), (11, 3), (12, 0), (13, 0), (14, 2), (17, 0),
                                       (22, 0), (23, 1)])
 def test_mobius_inverse_matches_oracle(backend, oracle, bits, off):
     from volta_mi355x import FP2

@@ -44,6 +44,9 @@ constexpr int MOBIUS_RUN_BITS = 3;  // Moebius passes above the first: at least 
 // One group of a full tile's four-bit round per thread; two tiles fit a CU's LDS,
 // four waves per SIMD.  2^21 points: 256 threads 43.1 us, 512 33.7, 1024 43.6.
 constexpr int MOBIUS_THREADS = 512;
+// One tile of up to 2^8 points has no work for the second half of them: 2^8 4.70 us with
+// 512 threads, 4.57 with 256; 2^9 5.0 and 5.1.
+constexpr int MOBIUS_SMALL_BITS = 8, MOBIUS_SMALL_THREADS = 256;
 constexpr uint64_t INV2 = 0x7FFFFFFF80000001ull;  // (p + 1) / 2
 using nreg::ROOT33_C1;
 using nreg::Digits;
@@ -143,11 +146,11 @@ __device__ __forceinline__ uint32_t mob_slot(uint32_t pc, uint32_t i, int rb) {
 // the middle index, all K of them in registers.  Group g takes the 2^K
 // elements of one (plane-column, the other bits of i); the bits' updates
 // commute, so any grouping of the bits gives the same result.
-template <int K>
+template <int K, int T>
 __device__ __forceinline__ void mobius_round(uint64_t* s, int b, int rb, uint32_t planecols, int inverse) {
     const uint32_t lo_mask = (1u << b) - 1, hi_bits = static_cast<uint32_t>(rb - b - K);
     const uint32_t groups = planecols << (rb - K);
-    for (uint32_t g = threadIdx.x; g < groups; g += MOBIUS_THREADS) {
+    for (uint32_t g = threadIdx.x; g < groups; g += T) {
         const uint32_t lo = g & lo_mask, hi = (g >> b) & ((1u << hi_bits) - 1), pc = g >> (rb - K);
         const uint32_t i0 = lo + (hi << (b + K));
         uint64_t v[1 << K];
@@ -173,7 +176,8 @@ __device__ __forceinline__ void mobius_round(uint64_t* s, int b, int rb, uint32_
 // bit of i, the element with the bit set gains (inverse) or loses the one
 // without.  Workgroup (h, l0) takes C = 2^cb adjacent columns; the bits are
 // applied up to four at a time in registers, with the tile in LDS in between.
-__global__ __launch_bounds__(MOBIUS_THREADS) void mobius_pass(u64x2* a, int rb, int lb, int cb, int inverse) {
+template <int T>
+__global__ __launch_bounds__(T) void mobius_pass(u64x2* a, int rb, int lb, int cb, int inverse) {
     extern __shared__ uint64_t s[];
     const uint32_t C = 1u << cb;
     const uint32_t CR = C << rb;
@@ -181,7 +185,7 @@ __global__ __launch_bounds__(MOBIUS_THREADS) void mobius_pass(u64x2* a, int rb, 
     const uint64_t h = blockIdx.x / lblocks;
     const uint64_t l0 = (blockIdx.x - h * lblocks) << cb;
     const uint64_t base = ((h << rb) << lb) + l0;
-    for (uint32_t e = threadIdx.x; e < CR; e += MOBIUS_THREADS) {
+    for (uint32_t e = threadIdx.x; e < CR; e += T) {
         const uint32_t i = e >> cb, c = e & (C - 1);
         const u64x2 v = a[base + (static_cast<uint64_t>(i) << lb) + c];
         s[mob_slot(c, i, rb)] = v.x;
@@ -190,14 +194,14 @@ __global__ __launch_bounds__(MOBIUS_THREADS) void mobius_pass(u64x2* a, int rb, 
     __syncthreads();
     for (int b = 0; b < rb; b += 4) {
         switch (rb - b >= 4 ? 4 : rb - b) {
-            case 4: mobius_round<4>(s, b, rb, 2 * C, inverse); break;
-            case 3: mobius_round<3>(s, b, rb, 2 * C, inverse); break;
-            case 2: mobius_round<2>(s, b, rb, 2 * C, inverse); break;
-            default: mobius_round<1>(s, b, rb, 2 * C, inverse); break;
+            case 4: mobius_round<4, T>(s, b, rb, 2 * C, inverse); break;
+            case 3: mobius_round<3, T>(s, b, rb, 2 * C, inverse); break;
+            case 2: mobius_round<2, T>(s, b, rb, 2 * C, inverse); break;
+            default: mobius_round<1, T>(s, b, rb, 2 * C, inverse); break;
         }
         __syncthreads();
     }
-    for (uint32_t e = threadIdx.x; e < CR; e += MOBIUS_THREADS) {
+    for (uint32_t e = threadIdx.x; e < CR; e += T) {
         const uint32_t i = e >> cb, c = e & (C - 1);
         a[base + (static_cast<uint64_t>(i) << lb) + c] = u64x2{s[mob_slot(c, i, rb)], s[mob_slot(C + c, i, rb)]};
     }
@@ -331,9 +335,15 @@ int fp2_mobius(Context* c, gl::Fp2* values, uint64_t n, bool inverse) {
         const size_t words = size_t{2} << (rb + cb);  // two planes
         const size_t lds = (words + (words >> 4) + 1 + (size_t{8} << cb)) * sizeof(uint64_t);  // + the slots' padding
         if (blocks > 0x7FFFFFFFull) return fail_msg(c, "Moebius pass exceeds its launch limits");
-        if (set_lds(c, mobius_pass, lds)) return -1;
-        hipLaunchKernelGGL(mobius_pass, dim3(static_cast<unsigned>(blocks)), dim3(MOBIUS_THREADS), lds, c->stream, a, rb,
-                           lb, cb, inverse ? 1 : 0);
+        auto launch = [&](auto kernel, int threads) {
+            if (set_lds(c, kernel, lds)) return -1;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds, c->stream, a, rb, lb, cb,
+                               inverse ? 1 : 0);
+            return 0;
+        };
+        if (nb <= MOBIUS_SMALL_BITS ? launch(mobius_pass<MOBIUS_SMALL_THREADS>, MOBIUS_SMALL_THREADS)
+                                    : launch(mobius_pass<MOBIUS_THREADS>, MOBIUS_THREADS))
+            return -1;
         VMX_HIP(c, hipGetLastError());
         done += rb;
         ++pass;
