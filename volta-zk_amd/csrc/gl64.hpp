@@ -14,7 +14,7 @@
 // add_lazy take 4 instructions (5 before), the general multiply 18 (20).  With
 // that, lazy sums inside the DFTs and the cheap negative of the middle shifts
 // (gl64_shift.hpp) a 32-point DFT takes 1,033 instead of 1,267 and a 16-point
-// one 397 instead of 483; measured alternating on one box: 2^15-point rows (C4)
+// one 397 instead of 483; measured alternating: 2^15-point rows (C4)
 // 4.47 -> 3.83 ms, the C3 step 1.674 -> 1.547 ms, C1 38.0 -> 35.9 us, the
 // 2^17-point embedding commitment 2.77 -> 2.65 ms; the 2^24-point batch only
 // 25.9 -> 25.4 ms, whose passes then wait on HBM.

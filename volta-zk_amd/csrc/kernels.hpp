@@ -44,7 +44,8 @@ int ntt13r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, s
                     TwiddleSet* t);
 int ntt14r_u64_rows(Context* c, const uint64_t* in, size_t stride, size_t len, size_t rows, size_t n, uint64_t* out,
                     TwiddleSet* t);
-// The same for message rows lift(w) || pads || 0 of either size.
+// The same for message rows lift(w) || pads || 0 of either size; 1 (nothing done) for
+// others and for batches too small to fill the chip with one workgroup per row.
 int ntt_rr_msg_rows(Context* c, const int16_t* w, const uint64_t* pads, size_t cols, size_t pad, size_t rows, size_t n,
                     uint64_t* out, TwiddleSet* t);
 // Rows of n = 2^8 .. 2^12 in one pass (ntt_small.hip): u64 rows as above, forward or

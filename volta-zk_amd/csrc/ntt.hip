@@ -4,9 +4,12 @@
 // out[j] = sum_i a_i w^(ij), w = 7^((p-1)/n), natural-order output.  Field sums
 // are exact, so any factorisation of the DFT gives bit-identical results.
 //
-// Rows of n >= 2^13 (u64, Fp2, and i16 weights + pads message rows) run on the
-// pass engine of ntt_reg.hip (register four-steps with shift-only sub-DFTs).
-// The generic path below serves smaller rows (any power-of-two n <= 2^14): one
+// Most rows of 2^13, 2^14 and 2^15 points (forward u64, and batches of i16 weights +
+// pads message rows) take one pass over HBM (ntt_rr.hip, ntt15.hip); Fp2 rows and all
+// others of n >= 2^13 run on the pass engine of ntt_reg.hip (register four-steps with
+// shift-only sub-DFTs).  Rows of 2^8 to 2^12 points run in one register pass
+// (ntt_small.hip; below 2^12 points, batches of at least 2^20).
+// The generic path below serves the rest (any power-of-two n <= 2^14): one
 // workgroup per row, the whole row in LDS (<= 128 KiB of the 160 KiB per CU),
 // bit-reversed load then radix-2^2 DIT passes (two stages per LDS round trip).
 // One HBM read + one HBM write per element.

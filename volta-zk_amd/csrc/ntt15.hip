@@ -48,7 +48,7 @@ __global__ __launch_bounds__(THREADS) void ntt15_rows(Src src, size_t rows, cons
     // last barrier and the next row's first one the waves run apart, and the
     // ones storing go first (2), then the ones loading and in stage A (1),
     // before any wave in the exchanges (0).  C4 4.85-4.93 -> 4.70-4.76 ms,
-    // p15 3.80-3.86 -> 3.72-3.78 ms, alternating on one box.
+    // p15 3.80-3.86 -> 3.72-3.78 ms, alternating.
     __builtin_amdgcn_s_setprio(1);
     for (; row < rows; row += gridDim.x) {
         // The role indices are recomputed from an opaque copy of the thread

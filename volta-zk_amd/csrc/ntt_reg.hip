@@ -142,7 +142,7 @@ constexpr int parked() {  // outputs per step-1 job in LDS at a time
 // is computed after this point instead of being held in registers across it.  The
 // two-round kernels otherwise keep step 2's addresses through step 1 and spill (13
 // words in the u64 gather, 4 in the column pass without a table): 2^18 x 16 rows,
-// gather 30 -> 24.3 us with no scratch.
+// gather 27.6 -> 24.5 us with no scratch.
 __device__ __forceinline__ uint32_t here() {
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));

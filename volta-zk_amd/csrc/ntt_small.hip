@@ -11,7 +11,8 @@
 // rows), 16 per thread, which cross LDS twice (34 KiB, four workgroups per CU).
 // The LDS kernel it takes over from (ntt_row_lds) runs B / 2 + 4 radix-2^2 rounds
 // through LDS with three general multiplies per four elements each.
-// VALU-issue bound on large batches (about 4.8 TB/s of loads and stores dense).
+// Bound by VALU issue on large batches from 2^9 points on (0.88-0.89 of the cycles; 4.84
+// TB/s of loads and stores dense at 2^12), by HBM at 2^8 (0.72; 5.56 TB/s).
 // Before (ntt_row_lds) and now, us, at 2^26 points: n = 2^8 321 / 193, 2^9 347 / 196,
 // 2^10 392 / 200, 2^11 449 / 209, 2^12 485 / 222; with the last three quarters of each
 // row zero 301 / 150, 322 / 167, 363 / 172, 405 / 182, 446 / 191.
